@@ -28,7 +28,7 @@
 
 #include <unistd.h>
 
-#include "dr_kernels.hpp"
+#include "dr_lines.hpp"
 
 namespace drh {
 
@@ -318,6 +318,28 @@ struct Chain : public ChainBase {
     DR_HIP(hipGetLastError());
     mark();
   }
+  // y or z pass of c2r_region / r2c_region between plain arrays: the register
+  // line kernels where there is one for the length (dr_lines.hpp) unless
+  // set_tuning asked for a tile or radix order of the kernels of dr_fft.hpp.
+  // Axis a, NB contiguous columns per outer index.
+  bool lines_ok(int a, int pid) const {
+    return (pid < 0 || tune_tbs[pid] < 0) && tune_order[a] == 0 && Nh * (long)sizeof(cx<T>) < (1L << 31);
+  }
+  template <bool INV>
+  void line_pass(int a, int n_outer, int NB, int k_in, int k_out, const cx<T>* src, long s_so, cx<T>* dst, long d_so,
+                 int pid = -1) {
+    const AxisFFT<T>& ad = axis_dev<T>(a);
+    DR_REQUIRE(k_in >= 1 && k_in <= ad.M && k_out >= 1 && k_out <= ad.M && NB >= 1 && n_outer >= 1, DR_ELOGIC,
+               "line pass: bad extents");
+    if (lines_ok(a, pid)) {
+      const LineArgs<T> la{ad.tw, NB, NB * n_outer, k_in, k_out, src, s_so, dst, d_so};
+      if (INV ? lines_inverse(ad.M, la, stream) : lines_forward(ad.M, la, stream)) {
+        mark();
+        return;
+      }
+    }
+    strided<T, INV>(a, n_outer, NB, k_in, k_out, LoadS<T>{{}, src, s_so, NB}, StoreS<T>{{}, dst, d_so, NB}, -1, pid);
+  }
   template <typename U, class Pro, class Epi>
   void xr2c(int nrows, Pro pro, Epi epi, int slot = -1, int pid = -1) {
     const AxisFFT<U> ad = axis_dev<U>(0);
@@ -486,21 +508,19 @@ struct Chain : public ChainBase {
                      StoreS<T>{{}, T2.p, (long)M[1] * H0, H0});
     xc2r<T>(M[1] * M[2], LoadRowC<T>{{}, T2.p, H0}, StoreRowR<T>{{}, dst, M[0], (T)(1.0 / (double)N)});
   }
-  // inverse transform pruned to the image region; Pro is the z-pass prologue
-  template <class Pro>
-  void c2r_region(Pro pro, T* R) {
-    strided<T, true>(2, 1, M[1] * H0, M[2], reg[2], pro, StoreS<T>{{}, T1.p, 0, (long)M[1] * H0});
-    strided<T, true>(1, reg[2], H0, M[1], reg[1], LoadS<T>{{}, T1.p, (long)M[1] * H0, H0},
-                     StoreS<T>{{}, T2.p, (long)reg[1] * H0, H0});
-    xc2r<T>(reg[1] * reg[2], LoadRowC<T>{{}, T2.p, H0}, StoreRowR<T>{{}, R, reg[0], (T)(1.0 / (double)N)});
+  // inverse transform of X pruned to the image region
+  void c2r_region(const cx<T>* X, T* R) {
+    z_inverse(X);
+    c2r_yx(R);
   }
+  // inverse z pass of X into T1 (z < n2)
+  void z_inverse(const cx<T>* X) { line_pass<true>(2, 1, M[1] * H0, M[2], reg[2], X, 0, T1.p, 0); }
   // forward transform from the image region; Pro is the x-pass prologue,
   // Epi the z-pass epilogue
   template <class Pro, class Epi>
   void r2c_region(Pro pro, Epi epi, int pro_slot, int epi_slot) {
     xr2c<T>(reg[1] * reg[2], pro, StoreRowC<T>{{}, T2.p, H0}, pro_slot);
-    strided<T, false>(1, reg[2], H0, reg[1], M[1], LoadS<T>{{}, T2.p, (long)reg[1] * H0, H0},
-                      StoreS<T>{{}, T1.p, (long)M[1] * H0, H0});
+    line_pass<false>(1, reg[2], H0, reg[1], M[1], T2.p, (long)reg[1] * H0, T1.p, (long)M[1] * H0);
     strided<T, false>(2, 1, M[1] * H0, reg[2], M[2], LoadS<T>{{}, T1.p, 0, (long)M[1] * H0}, epi, epi_slot);
   }
   // full-torus noise field -> spectral momentum (or initial mu)
@@ -1438,28 +1458,73 @@ struct Chain : public ChainBase {
   }
   // inverse y and x passes from T1 (z < n2) to the real region field R
   void c2r_yx(T* R) {
-    strided<T, true>(1, reg[2], H0, M[1], reg[1], LoadS<T>{{}, T1.p, (long)M[1] * H0, H0},
-                     StoreS<T>{{}, T2.p, (long)reg[1] * H0, H0}, -1, P_YI);
+    y_inverse();
+    if (lines_ok(0, P_XI) && rows_c2r(M[0] / 2, row_args(R), stream)) {
+      mark();
+      return;
+    }
     xc2r<T>(reg[1] * reg[2], LoadRowC<T>{{}, T2.p, H0}, StoreRowR<T>{{}, R, reg[0], (T)(1.0 / (double)N)}, -1,
             P_XI);
   }
   // forward x and y passes of the scattered residual into T1 (z < n2)
   void r2c_xy(LoadResidual<T> pro, int pro_slot) {
-    xr2c<T>(reg[1] * reg[2], pro, StoreRowC<T>{{}, T2.p, H0}, pro_slot, P_XF);
-    strided<T, false>(1, reg[2], H0, reg[1], M[1], LoadS<T>{{}, T2.p, (long)reg[1] * H0, H0},
-                      StoreS<T>{{}, T1.p, (long)M[1] * H0, H0}, -1, P_YF);
+    const int g = lines_ok(0, P_XF) ? rows_r2c(M[0] / 2, row_args(nullptr), pro, stream) : 0;
+    if (g) {
+      if (pro_slot >= 0) note_blocks(pro_slot, g);
+      mark();
+    } else {
+      xr2c<T>(reg[1] * reg[2], pro, StoreRowC<T>{{}, T2.p, H0}, pro_slot, P_XF);
+    }
+    y_forward();
+  }
+  // inverse y and x passes, the likelihood at the samples and its residual
+  // transformed back into T1.  A single-resolution residual is local to a row
+  // and takes one kernel on T2 in place, which writes mu to R only if keep.
+  void likelihood(T* R, int slot_h, int slot_s, bool keep) {
+    if (cfg.n_datasets == 1 && lines_ok(0, P_XI) && lines_ok(0, P_XF)) {
+      y_inverse();
+      if (const int g = rows_residual(M[0] / 2, row_args(keep ? R : nullptr), residual(R, slot_h), stream)) {
+        if (slot_h >= 0) note_blocks(slot_h, g);
+        mark();
+        mark();  // the inverse and forward x passes of the profile
+        y_forward();
+        return;
+      }
+      xc2r<T>(reg[1] * reg[2], LoadRowC<T>{{}, T2.p, H0}, StoreRowR<T>{{}, R, reg[0], (T)(1.0 / (double)N)}, -1,
+              P_XI);
+    } else {
+      c2r_yx(R);
+    }
+    w_products(R, slot_s);
+    r2c_xy(residual(R, slot_h), slot_h);
+  }
+  RowArgs<T> row_args(T* R) {
+    return RowArgs<T>{axis_dev<T>(0).tw, reg[1] * reg[2], reg[0], T2.p, T2.p, R, (T)(1.0 / (double)N)};
+  }
+  void y_inverse() {
+    line_pass<true>(1, reg[2], H0, M[1], reg[1], T1.p, (long)M[1] * H0, T2.p, (long)reg[1] * H0, P_YI);
+  }
+  void y_forward() {
+    line_pass<false>(1, reg[2], H0, reg[1], M[1], T2.p, (long)reg[1] * H0, T1.p, (long)M[1] * H0, P_YF);
   }
   // forward z pass, kick + drift, inverse z pass, in place on T1
   void zfused(MidLeapfrog<T> mid, int mid_slot) {
     const AxisFFT<T>& ad = axis_dev<T>(2);
     const int NB = M[1] * H0;
+    DR_REQUIRE(reg[2] >= 1 && reg[2] <= ad.M && NB >= 1, DR_ELOGIC, "z pass: bad extents");
+    if (lines_ok(2, P_Z)) {
+      if (const int g = lines_z(ad.M, ad.tw, NB, reg[2], reg[2], T1.p, mid, stream)) {
+        if (mid_slot >= 0) note_blocks(mid_slot, g);
+        mark();
+        return;
+      }
+    }
     const int tbs = tuned_tbs(P_Z, pick_tbs(ad.M, ad.M, sizeof(cx<T>), false, NB, kTileStrided),
                               pick_tbs(ad.M, ad.M, sizeof(cx<T>), false, 1 << 20, kTileStrided));
     const int TB = 1 << tbs;
     const int grid = cdiv(NB, TB);
     const size_t lds = (size_t)ad.M * TB * sizeof(cx<T>);
     // the tile holds ad.M rows, of which the first reg[2] are loaded
-    DR_REQUIRE(reg[2] >= 1 && reg[2] <= ad.M && NB >= 1, DR_ELOGIC, "z pass: bad extents");
     if (mid_slot >= 0) note_blocks(mid_slot, grid);
     const long sk = (long)M[1] * H0;
     with_fft_len(ad.M, [&](auto mc) {
@@ -1494,9 +1559,8 @@ struct Chain : public ChainBase {
   // energy at A and B, the kinetic energy at the end and both SSEs.
   void leapfrog_core(double eps, int L) {
     const long sk = (long)M[1] * H0;
-    c2r_region(LoadS<T>{{}, muA.p, 0, sk}, RA.p);
-    w_products(RA.p, S_SSES_A);
-    r2c_xy(residual(RA.p, S_SSEH_A), S_SSEH_A);
+    z_inverse(muA.p);
+    likelihood(RA.p, S_SSEH_A, S_SSES_A, true);
     for (int s = 0; s < L; ++s) {
       const bool last = s == L - 1;
       if (prof && L >= 2 && s == 1) DR_HIP(hipEventRecord(ev[0], stream));
@@ -1507,9 +1571,7 @@ struct Chain : public ChainBase {
       MidLeapfrog<T> mid{s == 0 ? muA.p : muB.p, muB.p, p.p, invlam.p, sk, (T)((s == 0 ? 0.5 : 1.0) * eps),
                          (T)eps, (T)sigma[0], H0, s == 0 ? 1 : 0, pslot(S_PRIOR_A), 0.0, gsc, s == 0 ? 0 : 1};
       zfused(mid, s == 0 ? S_PRIOR_A : -1);
-      c2r_yx(RB.p);
-      w_products(RB.p, last ? S_SSES_B : -1);
-      r2c_xy(residual(RB.p, last ? S_SSEH_B : -1), last ? S_SSEH_B : -1);
+      likelihood(RB.p, last ? S_SSEH_B : -1, last ? S_SSES_B : -1, last);
       if (rec >= 0) {
         nrec = rec;
         rec = -1;
@@ -1869,8 +1931,7 @@ struct Chain : public ChainBase {
   void refresh_stats() override {
     if (stats_valid) return;
     clear_slots();
-    const long sk = (long)M[1] * H0;
-    c2r_region(LoadS<T>{{}, muA.p, 0, sk}, RA.p);
+    c2r_region(muA.p, RA.p);
     quad(muA.p, S_PRIOR_A, (T)-1);
     if (compat()) quad(miA.p, S_PRIORI_A, (T)-1);
     if (data_set) {
@@ -1964,7 +2025,7 @@ struct Chain : public ChainBase {
     DR_REQUIRE(data_set, DR_ELOGIC, "gradient: data not set");
     if (Rf.n != (size_t)N) Rf.alloc(N);
     const long sk = (long)M[1] * H0;
-    c2r_region(LoadS<T>{{}, muA.p, 0, sk}, RA.p);
+    c2r_region(muA.p, RA.p);
     w_products(RA.p, -1);
     r2c_region(residual(RA.p, -1), EpiGrad<T>{{}, muA.p, muB.p, invlam.p, sk}, -1, -1);
     c2r_full(muB.p, Rf.p);

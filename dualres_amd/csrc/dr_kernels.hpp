@@ -154,21 +154,26 @@ template <typename T> struct MidLeapfrog {
   // the state one mode's update reads; each mode is read and written by one
   // thread only, so a thread may fetch its modes' state early
   struct State { cx<T> x, p; T il; };
-  __device__ __forceinline__ State fetch(int k, int b) const {
-    const long i = (long)k * sk + b;
+  template <class I> __device__ __forceinline__ State fetch_at(I i) const {
     // 1/lambda keeps cached loads: a 16-column tile reads half of each of its
     // 128-byte lines, and the neighbouring tile the other half
     return State{nt_ld(X + i), nt_ld(p + i), invlam[i]};
   }
-  __device__ __forceinline__ cx<T> apply(int k, int b, cx<T> v, const State& s) {
-    const long i = (long)k * sk + b;
+  // mode i of column b; write = false leaves memory and the sum alone
+  template <class I> __device__ __forceinline__ cx<T> apply_at(I i, int b, cx<T> v, const State& s, bool write) {
     const cx<T> pn = s.p + (v - s.x * s.il) * coef;
-    nt_st(p + i, pn);
     const T c = s.il > (T)0 ? eps / (s.il + sig) : (T)0;
     const cx<T> m = s.x + pn * c;
-    nt_st(Xd + i, m);
-    if (do_red) a0 += herm_w(b % H0, H0) * (double)s.il * ((double)s.x.x * s.x.x + (double)s.x.y * s.x.y);
+    if (write) {
+      nt_st(p + i, pn);
+      nt_st(Xd + i, m);
+      if (do_red) a0 += herm_w(b % H0, H0) * (double)s.il * ((double)s.x.x * s.x.x + (double)s.x.y * s.x.y);
+    }
     return m;
+  }
+  __device__ __forceinline__ State fetch(int k, int b) const { return fetch_at((long)k * sk + b); }
+  __device__ __forceinline__ cx<T> apply(int k, int b, cx<T> v, const State& s) {
+    return apply_at((long)k * sk + b, b, v, s, true);
   }
   __device__ __forceinline__ cx<T> apply(int k, int b, cx<T> v) { return apply(k, b, v, fetch(k, b)); }
   __device__ __forceinline__ void finish(double* red, int blk) {

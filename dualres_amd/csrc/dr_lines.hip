@@ -1,0 +1,104 @@
+// Instances of the register line transforms (dr_lines.hpp) for every length
+// of DR_LINE_LENGTHS.  Compiled once per precision and pass (DR_LINES_T;
+// DR_LINES_PASS 0 inverse strided, 1 forward strided, 2 leapfrog z, 3 rows
+// without the residual, 4 rows with it) so the objects build side by side.
+#include "dr_lines.hpp"
+
+namespace drh {
+
+using LT = DR_LINES_T;
+
+#if DR_LINES_PASS == 2
+int lines_z(int M, const cx<LT>* tw, int nb, int n_in, int n_out, cx<LT>* T1, const MidLeapfrog<LT>& mid,
+            hipStream_t s) {
+#define DR_CASE(m)                                                                                       \
+  case m: {                                                                                              \
+    using Sh = ZShape<LT, m>;                                                                         \
+    const int g = cdiv(nb, Sh::TB);                                                                      \
+    hipLaunchKernelGGL((k_zlines<LT, m>), dim3(g), dim3(Sh::NT), 0, s, tw, nb, n_in, n_out, T1, mid);    \
+    DR_HIP(hipGetLastError());                                                                           \
+    return g;                                                                                            \
+  }
+  switch (M) {
+    DR_LINE_LENGTHS(DR_CASE)
+    default: return 0;
+  }
+#undef DR_CASE
+}
+#elif DR_LINES_PASS < 2
+#if DR_LINES_PASS == 0
+int lines_inverse(int M, const LineArgs<LT>& a, hipStream_t s) {
+#else
+int lines_forward(int M, const LineArgs<LT>& a, hipStream_t s) {
+#endif
+#define DR_CASE(m)                                                                                       \
+  case m: {                                                                                              \
+    using Sh = StridedShape<LT, m>;                                                                         \
+    const int g = cdiv(a.ncol, Sh::TB);                                                                  \
+    hipLaunchKernelGGL((k_lines<LT, DR_LINES_PASS == 0, m>), dim3(g), dim3(Sh::NT), 0, s, a);            \
+    DR_HIP(hipGetLastError());                                                                           \
+    return g;                                                                                            \
+  }
+  switch (M) {
+    DR_LINE_LENGTHS(DR_CASE)
+    default: return 0;
+  }
+#undef DR_CASE
+}
+#else
+// rows: the table lists M0 = 2 Mh
+#define DR_ROWS(KERNEL, ...)                                                                             \
+  {                                                                                                      \
+    using Sh = RowShape<LT, MH>;                                                                         \
+    const int g = cdiv(a.nrows, Sh::RW);                                                                 \
+    hipLaunchKernelGGL((KERNEL<LT, MH>), dim3(g), dim3(Sh::NT), 0, s, __VA_ARGS__);                      \
+    DR_HIP(hipGetLastError());                                                                           \
+    return g;                                                                                            \
+  }
+#if DR_LINES_PASS == 3
+int rows_c2r(int Mh, const RowArgs<LT>& a, hipStream_t s) {
+#define DR_CASE(m)                     \
+  case m: {                            \
+    constexpr int MH = m / 2;          \
+    DR_ROWS(k_c2r_rows, a)             \
+  }
+  switch (2 * Mh) {
+    DR_LINE_LENGTHS(DR_CASE)
+    default: return 0;
+  }
+#undef DR_CASE
+}
+int rows_r2c(int Mh, const RowArgs<LT>& a, const LoadResidual<LT>& res, hipStream_t s) {
+  if (a.n0 < 2) return 0;  // samples are fetched in pairs
+  const RowResidual<LT> rr{res};
+#define DR_CASE(m)                     \
+  case m: {                            \
+    constexpr int MH = m / 2;          \
+    DR_ROWS(k_r2c_rows, a, rr)         \
+  }
+  switch (2 * Mh) {
+    DR_LINE_LENGTHS(DR_CASE)
+    default: return 0;
+  }
+#undef DR_CASE
+}
+#else
+int rows_residual(int Mh, const RowArgs<LT>& a, const LoadResidual<LT>& res, hipStream_t s) {
+  if (a.n0 < 2) return 0;  // samples are fetched in pairs
+  const RowResidual<LT> rr{res};
+#define DR_CASE(m)                     \
+  case m: {                            \
+    constexpr int MH = m / 2;          \
+    DR_ROWS(k_residual_rows, a, rr)    \
+  }
+  switch (2 * Mh) {
+    DR_LINE_LENGTHS(DR_CASE)
+    default: return 0;
+  }
+#undef DR_CASE
+}
+#endif
+#undef DR_ROWS
+#endif
+
+}  // namespace drh
