@@ -6,19 +6,29 @@
 //     position-sensitive hash per row.
 //  2. Host: rows with equal (count, hash) share one kriging system; equality
 //     is then verified element by element on the device (k_verify).
-//  3. Unique systems, sorted by size and padded with an identity block to a
-//     multiple of 64, are factorised in batches by a blocked left-looking
+//  3. Every system is K[S, S] w = k' for the offsets S present around a row,
+//     K the kernel matrix of the whole ball.  With B = K^-1 and D the absent
+//     offsets, w extended by zeros on D is (k' + y) B, where y lives on D and
+//     B[D, D] y = -(k' B)[D].  So one inverse, two products of all systems
+//     with B on the FP64 matrix cores and a Cholesky of |D| unknowns replace
+//     one of |S|; a refinement step (the residual on S, the same solve again)
+//     leaves the result as accurate as the direct solve.  A system with
+//     |S| < |D| is solved directly.  At 1 mm (balls of 1,357, rows at the
+//     mask's edge lose up to half of theirs) this is a few per cent of the
+//     direct factorisations' work.
+//     The batches, sorted by size and padded with an identity block to a
+//     multiple of 64, are factorised by a blocked left-looking
 //     float64 Cholesky over 64x64 tiles, two launches per tile
 //     column: k_chol_diag subtracts the finished columns' products from the
 //     diagonal tile, factors it and inverts the factor; k_chol_panel does
 //     the same subtraction for the tiles below and multiplies them by that
 //     inverse (the products on the FP64 matrix cores).  Then solved by tiles
 //     with those inverses (k_solve_chol), then
-//     normalised by their sum (kriging_matrix.h:318-321).  Systems whose
-//     Cholesky meets a nonpositive pivot (K with its unit diagonal is
-//     indefinite when tau^2 > 1) are factorised again by a blocked LU with
-//     partial pivoting (k_getrf_panel / k_trsm_lu / k_gemm_lu_mfma) and
-//     solved by k_solve_lu.
+//     normalised by their sum (kriging_matrix.h:318-321).  If the Cholesky
+//     of K itself meets a nonpositive pivot (K with its unit diagonal is
+//     indefinite when tau^2 > 1), every system is solved directly, and those
+//     whose Cholesky fails too by a blocked LU with partial pivoting
+//     (k_getrf_panel / k_trsm_lu / k_gemm_lu_mfma, k_solve_lu).
 //  4. Rows gather their system's weights; rows whose weights sum to NaN stay
 //     empty, as in the reference.
 // K and k' entries are float32 (the reference evaluates rbf<float>), taken as
@@ -262,8 +272,10 @@ __device__ __forceinline__ void zero_acc(dr_v4f64 acc[2][2]) {
 // trailing tile once per panel).  The tile pair of panel l + 1 is fetched
 // into registers while the matrix cores work on panel l from LDS.  Returns
 // with every thread past its last read of Pi and Pj.
+// a0(i, c) is entry (BI + i, BJ + c) of A.
+template <class A0>
 __device__ __forceinline__ void col_update(const double* As, int np, int BI, int BJ, int j, Tile& Pi, Tile& Pj,
-                                           const TileLane& q, double cv[2][2][4]) {
+                                           const TileLane& q, double cv[2][2][4], A0&& a0) {
   const int lc = threadIdx.x & 63, lr = threadIdx.x >> 6;  // loads: column lc of rows lr + 4 r
   double gi[16], gj[16];
   auto fetch = [&](int l) {
@@ -278,7 +290,7 @@ __device__ __forceinline__ void col_update(const double* As, int np, int BI, int
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) cv[a][b][t] = As[(long)(BI + q.row(a, t)) * np + BJ + q.col(b)];
+      for (int t = 0; t < 4; ++t) cv[a][b][t] = a0(q.row(a, t), q.col(b));
   dr_v4f64 acc[2][2];
   zero_acc(acc);
   if (j > 0) fetch(0);
@@ -322,8 +334,9 @@ __device__ __forceinline__ double lane_value(double v, int l) {
 // One wavefront factors the 64x64 tile T in place, lane c holding row c in
 // registers: for j = 0..63, L[j][j] = sqrt(A[j][j]), L[c][j] = A[c][j] /
 // L[j][j] for c > j, then A[c][m] -= L[c][j] L[m][j] for m > j (rows c < m
-// update entries above the diagonal, which are never read).  Returns 1 on a
-// nonpositive pivot.
+// update entries above the diagonal, which are never read).  The values of
+// column j come by v_readlane; as broadcast reads of a copy in LDS they took
+// the same time.  Returns 1 on a nonpositive pivot.
 __device__ __forceinline__ int potrf_wave(Tile& T) {
   const int c = threadIdx.x & 63;
   double a[NB];
@@ -353,7 +366,7 @@ __device__ __forceinline__ int potrf_wave(Tile& T) {
 __device__ __forceinline__ void trtri_block(Tile& T, Tile& W) {
   for (int t = threadIdx.x; t < NB; t += 256) W[t][t] = 1.0 / T[t][t];
   __syncthreads();
-  for (int s = 1; s < NB; s *= 2) {
+  for (int s = 1; s < 16; s *= 2) {
     const int n = (NB / (2 * s)) * s * s;  // elements of all blocks at this level
     for (int t = threadIdx.x; t < n; t += 256) {  // U[cc][r] = (B A^-1)[r][cc]
       const int b = (t / (s * s)) * 2 * s, r = (t / s) % s, cc = t % s;
@@ -370,6 +383,41 @@ __device__ __forceinline__ void trtri_block(Tile& T, Tile& W) {
     }
     __syncthreads();
   }
+  // s = 16 and 32 on the matrix cores, a 16x16 block of a product per
+  // wavefront (as chains of dependent LDS reads they took half of the
+  // tile's time)
+  const int w = threadIdx.x >> 6, li = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int s = 16; s < NB; s *= 2) {
+    const int q = s / 16;  // blocks of 16 per side
+    const bool on = w < (NB / (2 * s)) * q * q;
+    const int b = w / (q * q) * 2 * s, r0 = (w / q) % q * 16, c0 = w % q * 16;
+    dr_v4f64 acc = dr_v4f64{0.0, 0.0, 0.0, 0.0};
+    if (on) {
+      for (int kk = 0; kk < s; kk += 4) {
+        const int k = kk + lk;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(T[b + s + r0 + li][b + k],
+                                                   k >= c0 + li ? W[b + k][b + c0 + li] : 0.0, acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) W[b + c0 + li][b + s + r0 + 4 * t + lk] = acc[t];
+    }
+    __syncthreads();
+    acc = dr_v4f64{0.0, 0.0, 0.0, 0.0};
+    if (on) {
+      for (int kk = 0; kk < s; kk += 4) {
+        const int k = kk + lk;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(k <= r0 + li ? W[b + s + r0 + li][b + s + k] : 0.0,
+                                                   W[b + c0 + li][b + s + k], acc, 0, 0, 0);
+      }
+    }
+    __syncthreads();
+    if (on) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) W[b + s + r0 + 4 * t + lk][b + c0 + li] = -acc[t];
+    }
+    __syncthreads();
+  }
   for (int t = threadIdx.x; t < NB * NB; t += 256) {
     const int i = t / NB, c = t % NB;
     if (i > c) T[c][i] = W[i][c];
@@ -383,41 +431,39 @@ __device__ __forceinline__ void lds_to_tile(const Tile& T, double* As, int np, i
   }
 }
 
-// Cholesky, tile column j, diagonal tile: update, factor, invert
-__global__ void __launch_bounds__(256) k_chol_diag(double* A, int np, int j, int* fail) {
-  __shared__ Tile Pi, Pj;
-  double* As = A + (long)blockIdx.x * np * np;
+// Cholesky, tile column j, diagonal tile: update, factor, invert; returns 1
+// (in the first wavefront) on a nonpositive pivot
+template <class A0>
+__device__ __forceinline__ int chol_diag_tile(double* As, int np, int j, Tile& Pi, Tile& Pj, A0&& a0) {
   const TileLane q;
   double cv[2][2][4];
-  col_update(As, np, j * NB, j * NB, j, Pi, Pj, q, cv);
+  col_update(As, np, j * NB, j * NB, j, Pi, Pj, q, cv, a0);
   cv_to_lds(cv, q, Pi);
   __syncthreads();
-  if (threadIdx.x < 64) {
-    const int bad = potrf_wave(Pi);
-    if (bad && threadIdx.x == 0) fail[blockIdx.x] = 1;
-  }
+  int bad = 0;
+  if (threadIdx.x < 64) bad = potrf_wave(Pi);
   __syncthreads();
   trtri_block(Pi, Pj);
   __syncthreads();
   lds_to_tile(Pi, As, np, j * NB, j * NB);
+  return bad;
 }
 
-// Cholesky, tile column j, the tile rows i = j + 1 + blockIdx.y below the
-// diagonal: update, then L[i][j] = C L[j][j]^-T as a product with the
-// inverse k_chol_diag left above the diagonal (in place of a
+// Cholesky, tile column j, tile row i > j: update, then
+// L[i][j] = C L[j][j]^-T as a product with the
+// inverse chol_diag_tile left above the diagonal (in place of a
 // column-by-column substitution, 64 dependent steps per tile)
-__global__ void __launch_bounds__(256) k_chol_panel(double* A, int np, int j) {
-  __shared__ Tile Pi, Pj;
-  double* As = A + (long)blockIdx.x * np * np;
-  const int BI = (j + 1 + blockIdx.y) * NB, o = j * NB;
+template <class A0>
+__device__ __forceinline__ void chol_panel_tile(double* As, int np, int i, int j, Tile& Pi, Tile& Pj, A0&& a0) {
+  const int BI = i * NB, o = j * NB;
   const TileLane q;
   double cv[2][2][4];
-  col_update(As, np, BI, o, j, Pi, Pj, q, cv);
+  col_update(As, np, BI, o, j, Pi, Pj, q, cv, a0);
   cv_to_lds(cv, q, Pi);
   const double* D = As + (long)o * np + o;
   for (int t = threadIdx.x; t < NB * NB; t += 256) {  // Pj[i][l] = L^-1[i][l]
-    const int i = t / NB, l = t % NB;
-    Pj[i][l] = l < i ? D[(long)l * np + i] : l == i ? 1.0 / D[(long)i * np + i] : 0.0;
+    const int l = t / NB, r = t % NB;
+    Pj[r][l] = l < r ? D[(long)l * np + r] : l == r ? 1.0 / D[(long)r * np + r] : 0.0;
   }
   __syncthreads();
   dr_v4f64 acc[2][2];
@@ -429,6 +475,279 @@ __global__ void __launch_bounds__(256) k_chol_panel(double* A, int np, int j) {
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int t = 0; t < 4; ++t) As[(long)(BI + q.row(a, t)) * np + o + q.col(b)] = acc[a][b][t];
+}
+
+// One tile column of every system of a batch in place (blockIdx.x; tile row
+// j + 1 + blockIdx.y): for few or very large systems, whose tile rows then
+// spread over the chip.
+__global__ void __launch_bounds__(256) k_chol_diag(double* A, int np, int j, int* fail) {
+  __shared__ Tile Pi, Pj;
+  double* As = A + (long)blockIdx.x * np * np;
+  const int o = j * NB;
+  const int bad = chol_diag_tile(As, np, j, Pi, Pj, [&](int i, int c) { return As[(long)(o + i) * np + o + c]; });
+  if (bad && threadIdx.x == 0) fail[blockIdx.x] = 1;
+}
+__global__ void __launch_bounds__(256) k_chol_panel(double* A, int np, int j) {
+  __shared__ Tile Pi, Pj;
+  double* As = A + (long)blockIdx.x * np * np;
+  const int i = j + 1 + blockIdx.y, BI = i * NB, o = j * NB;
+  chol_panel_tile(As, np, i, j, Pi, Pj, [&](int r, int c) { return As[(long)(BI + r) * np + o + c]; });
+}
+
+// ---------------------------------------------------------------- K and its inverse
+// K of the ball (kriging_matrix.h:111-138): unit diagonal, float rounding of
+// the kernel at the separately rounded float distance; Kd the same in float64
+// padded with the identity to ld
+__global__ void k_kernel_matrix(Geo g, const float* __restrict__ X, int ld, float* __restrict__ K,
+                                double* __restrict__ Kd) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
+  if (j >= ld) return;
+  double v = i == j ? 1.0 : 0.0;
+  if (i < g.nP && j < g.nP) {
+    if (i != j) {
+      float ss = 0.0f;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const float d = sub_rn(X[3 * i + c], X[3 * j + c]), q = mul_rn(d, d);
+        ss = c == 0 ? q : add_rn(ss, q);
+      }
+      v = (double)kern_f(g, sqrt_rn(ss));
+    }
+    K[(long)i * g.nP + j] = (float)v;
+  }
+  Kd[(long)i * ld + j] = v;
+}
+
+// Wt[c][i] = (L^-1)[i][c]^T from the factor and the inverses of its diagonal
+// tiles (k_chol_diag).  A column of L^-1 depends on itself alone, so a
+// workgroup walks down 16 of them (blockIdx.y of tile column blockIdx.x):
+// (L^-1)[i][c] = -L[i][i]^-1 sum_{c<=k<i} L[i][k] (L^-1)[k][c].  The walk is
+// a chain of tile products; 16 columns instead of 64 make it 4 times shorter
+// (2.2 ms at 1,357 offsets with 64).
+__global__ void __launch_bounds__(256) k_tri_inverse(const double* L, int np, double* Wt) {
+  constexpr int C = 16;
+  __shared__ Tile X;
+  __shared__ double Y[C][NB + 1];
+  const int c = blockIdx.x, nt = np / NB, c0 = c * NB + blockIdx.y * C;
+  const int w = threadIdx.x >> 6, li = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+  const int lc = threadIdx.x & 63, lr = threadIdx.x >> 6;
+  auto inv_diag = [&](int k) {  // X[i][l] = (L[k][k]^-1)[i][l]
+    const double* D = L + (long)(k * NB) * np + k * NB;
+    for (int t = threadIdx.x; t < NB * NB; t += 256) {
+      const int l = t / NB, i = t % NB;  // coalesced over the inverse's rows above the diagonal
+      X[i][l] = l < i ? D[(long)l * np + i] : l == i ? 1.0 / D[(long)i * np + i] : 0.0;
+    }
+  };
+  inv_diag(c);
+  __syncthreads();
+  for (int t = threadIdx.x; t < C * NB; t += 256)
+    Wt[(long)(c0 + t / NB) * np + c * NB + t % NB] = X[t % NB][blockIdx.y * C + t / NB];
+  __syncthreads();
+  double gx[16], gy[4];
+  auto fetch = [&](int i, int k) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) gx[r] = L[(long)(i * NB + lr + 4 * r) * np + k * NB + lc];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) gy[r] = Wt[(long)(c0 + lr + 4 * r) * np + k * NB + lc];  // this workgroup's own
+  };
+  for (int i = c + 1; i < nt; ++i) {
+    dr_v4f64 acc = dr_v4f64{0.0, 0.0, 0.0, 0.0};
+    fetch(i, c);
+    for (int k = c; k < i; ++k) {
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < 16; ++r) X[lr + 4 * r][lc] = gx[r];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) Y[lr + 4 * r][lc] = gy[r];
+      __syncthreads();
+      if (k + 1 < i) fetch(i, k + 1);
+#pragma unroll 4
+      for (int kk = 0; kk < NB; kk += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(X[16 * w + li][kk + lk], Y[li][kk + lk], acc, 0, 0, 0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 4; ++t) Y[li][16 * w + 4 * t + lk] = -acc[t];  // transposed
+    inv_diag(i);
+    __syncthreads();
+    acc = dr_v4f64{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int kk = 0; kk < NB; kk += 4)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(Y[li][kk + lk], X[16 * w + li][kk + lk], acc, 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) Wt[(long)(c0 + 4 * t + lk) * np + i * NB + 16 * w + li] = acc[t];
+    __syncthreads();  // read back in the next row's products
+  }
+}
+
+// C = X Y^T (plus C0 where given) by 64x64 tiles over kt tile columns from
+// max(blockIdx.x, blockIdx.y) when tri (both operands upper triangular), else
+// from 0; the next tile pair is fetched while the matrix cores work
+__global__ void __launch_bounds__(256) k_gemm_xyt(const double* __restrict__ X, const double* __restrict__ Y, int ld,
+                                                  int kt, int tri, const double* C0, double* C) {
+  __shared__ Tile Pi, Pj;
+  const int BI = blockIdx.y * NB, BJ = blockIdx.x * NB;
+  const int lc = threadIdx.x & 63, lr = threadIdx.x >> 6;
+  const TileLane q;
+  double gi[16], gj[16];
+  auto fetch = [&](int l) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      gi[r] = X[(long)(BI + lr + 4 * r) * ld + l * NB + lc];
+      gj[r] = Y[(long)(BJ + lr + 4 * r) * ld + l * NB + lc];
+    }
+  };
+  dr_v4f64 acc[2][2];
+  zero_acc(acc);
+  const int k0 = tri ? max((int)blockIdx.x, (int)blockIdx.y) : 0;
+  fetch(k0);
+  for (int l = k0; l < kt; ++l) {
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      Pi[lr + 4 * r][lc] = gi[r];
+      Pj[lr + 4 * r][lc] = gj[r];
+    }
+    __syncthreads();
+    if (l + 1 < kt) fetch(l + 1);
+    mfma_xyt(Pi, Pj, q, acc);
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const long o = (long)(BI + q.row(a, t)) * ld + BJ + q.col(b);
+        C[o] = C0 ? C0[o] + acc[a][b][t] : acc[a][b][t];
+      }
+}
+
+// ---------------------------------------------------------------- extended systems
+struct ExtDesc {
+  long off;  // entries of the representative row (pidx, k')
+  int n;     // present offsets
+  int m;     // absent ones
+  long dl;   // offset into the list of absent ones
+  long sol;  // offset into the solution buffer
+};
+// one factorisation: m unknowns at list (of B over absent offsets, or of K
+// over the present ones of a direct system), its factor, its extended row
+// (-1: direct) and a direct solution's place
+struct FacDesc {
+  int m, row;
+  long list, fac, sol;
+};
+
+// The whole Cholesky of B[D, D], or of K[S, S] for a direct system, per
+// workgroup, read straight from B or K (identity past m): systems of all
+// sizes share one launch, the largest first.  A launch per tile column and
+// size left most of the chip idle: some 60 us each for a few hundred systems
+// (kriging build at 48x60x48, 1 mm: 53 ms, 39 ms with one launch).
+__global__ void __launch_bounds__(256, 2) k_factor_all(const FacDesc* __restrict__ fd, const double* __restrict__ B,
+                                                       const double* __restrict__ K, int ld,
+                                                       const int* __restrict__ dlist, const int* __restrict__ pidx,
+                                                       double* A, int* fail) {
+  __shared__ Tile Pi, Pj;
+  const FacDesc d = fd[blockIdx.x];
+  const int nt = (d.m + NB - 1) / NB, np = nt * NB;
+  double* As = A + d.fac;
+  const int* id = (d.row < 0 ? pidx : dlist) + d.list;
+  const double* G = d.row < 0 ? K : B;
+  auto entry = [&](int r, int c) {
+    if (r >= d.m || c >= d.m) return r == c ? 1.0 : 0.0;
+    return G[(long)id[r] * ld + id[c]];
+  };
+  int bad = 0;
+  for (int j = 0; j < nt; ++j) {
+    const int o = j * NB;
+    bad |= chol_diag_tile(As, np, j, Pi, Pj, [&](int r, int c) { return entry(o + r, o + c); });
+    __syncthreads();  // the tile is read back below
+    for (int i = j + 1; i < nt; ++i) {
+      chol_panel_tile(As, np, i, j, Pi, Pj, [&](int r, int c) { return entry(i * NB + r, o + c); });
+      __syncthreads();
+    }
+  }
+  if (bad && threadIdx.x == 0) fail[blockIdx.x] = 1;
+}
+
+// row of the extended right-hand side: k' on the present offsets, 0 on the
+// absent ones, whose list is written in increasing order
+__global__ void __launch_bounds__(256) k_extend(const ExtDesc* __restrict__ ed, int nP, int ld,
+                                                const int* __restrict__ pidx, const float* __restrict__ kp,
+                                                double* __restrict__ K0, int* __restrict__ dlist) {
+  extern __shared__ unsigned int on[];  // bit per offset
+  const ExtDesc d = ed[blockIdx.x];
+  double* row = K0 + (long)blockIdx.x * ld;
+  const int nw = (nP + 31) / 32;
+  for (int i = threadIdx.x; i < nw; i += 256) on[i] = 0u;
+  for (int i = threadIdx.x; i < ld; i += 256) row[i] = 0.0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < d.n; i += 256) {
+    const int j = pidx[d.off + i];
+    row[j] = (double)kp[d.off + i];
+    atomicOr(&on[j >> 5], 1u << (j & 31));
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) {  // one wavefront compacts the zero bits
+    int base = 0;
+    for (int j0 = 0; j0 < nP; j0 += 64) {
+      const int j = j0 + (int)threadIdx.x;
+      const bool off = j < nP && !(on[j >> 5] >> (j & 31) & 1u);
+      const uint64_t bal = __ballot(off);
+      if (off) dlist[d.dl + base + __popcll(bal & ((1ULL << threadIdx.x) - 1ULL))] = j;
+      base += __popcll(bal);
+    }
+  }
+}
+
+// residual of the extended systems on the present offsets, 0 on the absent
+// ones: E = k' - W K with W K in KW, W's absent offsets 0 by construction
+__global__ void __launch_bounds__(256) k_residual_ext(const ExtDesc* __restrict__ ed, int ld,
+                                                      const int* __restrict__ pidx, const float* __restrict__ kp,
+                                                      const double* __restrict__ KW, double* __restrict__ E) {
+  const ExtDesc d = ed[blockIdx.x];
+  const double* kw = KW + (long)blockIdx.x * ld;
+  double* e = E + (long)blockIdx.x * ld;
+  for (int i = threadIdx.x; i < ld; i += 256) e[i] = 0.0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < d.n; i += 256) {
+    const int j = pidx[d.off + i];
+    e[j] = (double)kp[d.off + i] - kw[j];
+  }
+}
+
+// W on the absent offsets is 0 up to rounding: make it so
+__global__ void __launch_bounds__(256) k_clear_absent(const ExtDesc* __restrict__ ed, int ld,
+                                                      const int* __restrict__ dlist, double* __restrict__ W) {
+  const ExtDesc d = ed[blockIdx.x];
+  double* w = W + (long)blockIdx.x * ld;
+  for (int i = threadIdx.x; i < d.m; i += 256) w[dlist[d.dl + i]] = 0.0;
+}
+
+// largest diagonal entry of B (one workgroup): 1 / the smallest variance of an
+// offset given all others
+__global__ void __launch_bounds__(256) k_max_diag(const double* __restrict__ B, int n, int ld, double* __restrict__ out) {
+  __shared__ double m[256];
+  double v = 0.0;
+  for (int i = threadIdx.x; i < n; i += 256) {
+    const double b = B[(long)i * ld + i];
+    v = b <= v ? v : b;  // a NaN is kept
+  }
+  m[threadIdx.x] = v;
+  __syncthreads();
+  for (int st = 128; st > 0; st >>= 1) {
+    if ((int)threadIdx.x < st) {
+      const double o = m[threadIdx.x + st];
+      if (!(o <= m[threadIdx.x])) m[threadIdx.x] = o;
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) out[0] = m[0];
+}
+
+__global__ void k_zero_f64(long n, double* __restrict__ p) {
+  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = 0.0;
 }
 
 // ---------------------------------------------------------------- LU with partial pivoting
@@ -589,24 +908,34 @@ __device__ __forceinline__ void normalise_out(const double* y, int n, double* pa
   for (int i = threadIdx.x; i < n; i += 256) out[i] = y[i] / tot;
 }
 
+// weights of an extended system: W (plus dW where given) on the present
+// offsets, normalised
+__global__ void __launch_bounds__(256) k_finish_ext(const ExtDesc* __restrict__ ed, int ld,
+                                                    const int* __restrict__ pidx, const double* __restrict__ W,
+                                                    const double* __restrict__ dW, double* __restrict__ sol) {
+  extern __shared__ double y[];
+  __shared__ double part[4];
+  const ExtDesc d = ed[blockIdx.x];
+  const double* w = W + (long)blockIdx.x * ld;
+  const double* dw = dW ? dW + (long)blockIdx.x * ld : nullptr;
+  for (int i = threadIdx.x; i < d.n; i += 256) {
+    const int j = pidx[d.off + i];
+    y[i] = dw ? w[j] + dw[j] : w[j];
+  }
+  __syncthreads();
+  normalise_out(y, d.n, part, sol + d.sol);
+}
+
 // Cholesky: L L^T w = b by 64-row tiles, with the inverses of the diagonal
 // tiles that k_chol_diag left above their diagonals.  Forward, tile k:
 // r = b_k - sum_{l<k} L[k][l] y_l, y_k = L[k][k]^-1 r; backward:
 // r = y_k - sum_{l>k} L[l][k]^T x_l, x_k = L[k][k]^-T r.  Tiles past the
 // system's size are identity padding with a zero right-hand side and are
-// skipped.
-__global__ void __launch_bounds__(256) k_solve_chol(const double* A, int np, const SysDesc* __restrict__ sd,
-                                                    const double* __restrict__ bv, double* __restrict__ sol) {
-  extern __shared__ double y[];
-  __shared__ double part[4][NB];
-  __shared__ double rk[NB];
-  const int s = blockIdx.x;
-  const SysDesc d = sd[s];
-  const double* As = A + (long)s * np * np;
-  const int nt = (d.n + NB - 1) / NB, nn = nt * NB;
+// skipped.  y: the right-hand side on entry, the solution on return.
+__device__ __forceinline__ void chol_solve(const double* As, int np, int n, double* y, double (*part)[NB],
+                                           double* rk) {
+  const int nt = (n + NB - 1) / NB, nn = nt * NB;
   const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-  for (int i = threadIdx.x; i < nn; i += 256) y[i] = bv[(long)s * np + i];
-  __syncthreads();
   for (int k = 0; k < nt; ++k) {
     const int o = k * NB;
     const double* D = As + (long)o * np + o;
@@ -657,7 +986,46 @@ __global__ void __launch_bounds__(256) k_solve_chol(const double* A, int np, con
     if (q == 0) y[o + lane] = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
     __syncthreads();
   }
+}
+
+__global__ void __launch_bounds__(256) k_solve_chol(const double* A, int np, const SysDesc* __restrict__ sd,
+                                                    const double* __restrict__ bv, double* __restrict__ sol) {
+  extern __shared__ double y[];
+  __shared__ double part[4][NB];
+  __shared__ double rk[NB];
+  const int s = blockIdx.x;
+  const SysDesc d = sd[s];
+  for (int i = threadIdx.x; i < np; i += 256) y[i] = bv[(long)s * np + i];
+  __syncthreads();
+  chol_solve(A + (long)s * np * np, np, d.n, y, part, rk);
   normalise_out(y, d.n, &part[0][0], sol + d.sol);
+}
+
+// y on the absent offsets of an extended system with F B in U, to its row of
+// Y (0 elsewhere); a direct system's weights to sol (first pass only)
+__global__ void __launch_bounds__(256) k_solve_all(const FacDesc* __restrict__ fd, const double* A, int ld,
+                                                   const int* __restrict__ dlist, const double* __restrict__ U,
+                                                   double* __restrict__ Y, const float* __restrict__ kp,
+                                                   double* __restrict__ sol, int first) {
+  extern __shared__ double y[];
+  __shared__ double part[4][NB];
+  __shared__ double rk[NB];
+  const FacDesc d = fd[blockIdx.x];
+  const bool direct = d.row < 0;
+  if (direct && !first) return;
+  const int np = (d.m + NB - 1) / NB * NB;
+  const int* id = dlist + d.list;
+  const double* u = U + (long)max(d.row, 0) * ld;
+  double* yr = Y + (long)max(d.row, 0) * ld;
+  for (int i = threadIdx.x; i < np; i += 256)
+    y[i] = i >= d.m ? 0.0 : direct ? (double)kp[d.list + i] : -u[id[i]];
+  __syncthreads();
+  chol_solve(A + d.fac, np, d.m, y, part, rk);
+  if (direct) {
+    normalise_out(y, d.m, &part[0][0], sol + d.sol);
+    return;
+  }
+  for (int i = threadIdx.x; i < d.m; i += 256) yr[id[i]] = y[i];
 }
 
 // LU: L U w = b with b already permuted, L unit lower and U upper in A; a
@@ -763,11 +1131,6 @@ struct DBuf {
   void down(T* h, size_t n, hipStream_t s) { DR_HIP(hipMemcpyAsync(h, p, n * sizeof(T), hipMemcpyDeviceToHost, s)); }
 };
 
-float fsq(float a) {
-  const volatile float r = a * a;
-  return r;
-}
-
 }  // namespace
 
 // ---------------------------------------------------------------- host build
@@ -828,18 +1191,6 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
   g.nu = (double)(float)theta[2];
   g.eps0 = 1e-5f;
   g.nP = nP;
-  // K (kriging_matrix.h:111-138): unit diagonal
-  std::vector<float> K((size_t)nP * nP);
-  for (int i = 0; i < nP; ++i) {
-    K[(size_t)i * nP + i] = 1.0f;
-    for (int j = 0; j < i; ++j) {
-      const float d[3] = {X[3 * i] - X[3 * j], X[3 * i + 1] - X[3 * j + 1], X[3 * i + 2] - X[3 * j + 2]};
-      const float ss = (fsq(d[0]) + fsq(d[1])) + fsq(d[2]);
-      const float v = kern_f(g, sqrt_rn(ss));
-      K[(size_t)i * nP + j] = v;
-      K[(size_t)j * nP + i] = v;
-    }
-  }
   // highres bounding box and bounded nonzero index (nifti_manipulation.inl:210-275)
   auto pres = [](double v) { return !(std::isnan(v) || v == 0.0); };
   std::vector<uint8_t> present(nvox);
@@ -979,37 +1330,67 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
   for (int i = 0; i < n_rows; ++i)
     DR_REQUIRE(!bad[i], DR_ERUNTIME, "kriging_build: hash collision between distinct kriging systems");
 
-  // unique systems sorted by size, batched by padded size; Cholesky first,
-  // then LU with partial pivoting for the systems whose Cholesky failed
-  std::vector<int> order(nU);
-  std::iota(order.begin(), order.end(), 0);
-  std::sort(order.begin(), order.end(), [&](int a, int b) { return cnt[urow[a]] > cnt[urow[b]]; });
   std::vector<long> usol(nU);
   long solsz = 0;
   for (int u = 0; u < nU; ++u) { usol[u] = solsz; solsz += cnt[urow[u]]; }
   DBuf<double> d_sol(solsz);
-  DBuf<float> d_K((size_t)nP * nP);
-  d_K.up(K.data(), (size_t)nP * nP, s);
+  // K, its factor and its inverse
+  const int ld = cdiv(nP, NB) * NB, ntl = ld / NB;
+  DBuf<float> d_X(X.size()), d_K((size_t)nP * nP);
+  DBuf<double> d_Kd((size_t)ld * ld), d_L((size_t)ld * ld);
+  DBuf<int> d_fail(1);
+  d_X.up(X.data(), X.size(), s);
+  hipLaunchKernelGGL(k_kernel_matrix, dim3(cdiv(ld, 256), ld), dim3(256), 0, s, g, d_X.p, ld, d_K.p, d_Kd.p);
+  DR_HIP(hipGetLastError());
+  DR_HIP(hipMemcpyAsync(d_L.p, d_Kd.p, (size_t)ld * ld * sizeof(double), hipMemcpyDeviceToDevice, s));
+  DR_HIP(hipMemsetAsync(d_fail.p, 0, sizeof(int), s));
+  auto cholesky = [&](double* A, int B, int np) {
+    const int nt = np / NB;
+    for (int k = 0; k < nt; ++k) {
+      hipLaunchKernelGGL(k_chol_diag, dim3(B), dim3(256), 0, s, A, np, k, d_fail.p);
+      if (k + 1 < nt) hipLaunchKernelGGL(k_chol_panel, dim3(B, nt - k - 1), dim3(256), 0, s, A, np, k);
+      DR_HIP(hipGetLastError());
+    }
+  };
+  cholesky(d_L.p, 1, ld);
+  // K^-1 = (L^-1)^T L^-1 into d_B.  Systems go through it only where K is
+  // well conditioned: a diagonal entry of K^-1 above 1e4 (a variance given
+  // all others below 1e-4; it is at least 1 - tau^2) keeps the direct solves.
+  DBuf<double> d_B((size_t)ld * ld), d_mx(1);
+  {
+    DBuf<double> d_Wt((size_t)ld * ld);
+    hipLaunchKernelGGL(k_tri_inverse, dim3(ntl, NB / 16), dim3(256), 0, s, d_L.p, ld, d_Wt.p);
+    hipLaunchKernelGGL(k_gemm_xyt, dim3(ntl, ntl), dim3(256), 0, s, d_Wt.p, d_Wt.p, ld, ntl, 1,
+                       (const double*)nullptr, d_B.p);
+    hipLaunchKernelGGL(k_max_diag, dim3(1), dim3(256), 0, s, d_B.p, nP, ld, d_mx.p);
+    DR_HIP(hipGetLastError());
+    DR_HIP(hipStreamSynchronize(s));
+  }
+  int kfail = 0;
+  double bmax_diag = 0.0;
+  d_fail.down(&kfail, 1, s);
+  d_mx.down(&bmax_diag, 1, s);
+  DR_HIP(hipStreamSynchronize(s));
+  const bool via_inverse = !kfail && bmax_diag <= 1e4;
+  // Batches of equal padded size, largest first.
   const double budget = 6.0e9;  // bytes of factor scratch per batch
   DBuf<double> d_A, d_b;
   DBuf<SysDesc> d_sd;
-  DBuf<int> d_fail;
   size_t capA = 0, capB = 0, capS = 0;
-  auto solve_all = [&](const std::vector<int>& uids, bool lu) {
+  // systems (unique indices) solved directly; returns those whose Cholesky failed
+  auto solve_all = [&](std::vector<int> uids, bool lu) {
+    std::stable_sort(uids.begin(), uids.end(), [&](int a, int b) { return cnt[urow[a]] > cnt[urow[b]]; });
     std::vector<int> failed;
     size_t pos = 0;
     while (pos < uids.size()) {
-      const int n0 = cnt[urow[uids[pos]]];
-      const int np = ((n0 + NB - 1) / NB) * NB;
+      const int np = cdiv(cnt[urow[uids[pos]]], NB) * NB;
       const long per = (long)np * np * 8;
-      const int bmax = (int)std::max<long>(1, std::min<long>(4096, (long)(budget / per)));
+      const int bmax = (int)std::max<long>(1, std::min<long>(16384, (long)(budget / per)));
       std::vector<SysDesc> sd;
-      std::vector<int> bu;
-      while (pos < uids.size() && (int)sd.size() < bmax) {
-        const int u = uids[pos];
+      const size_t first = pos;
+      while (pos < uids.size() && (int)sd.size() < bmax && cdiv(cnt[urow[uids[pos]]], NB) * NB == np) {
+        const int u = uids[pos++];
         sd.push_back(SysDesc{rp[urow[u]], cnt[urow[u]], usol[u]});
-        bu.push_back(u);
-        ++pos;
       }
       const int B = (int)sd.size();
       if ((size_t)B * np * np > capA) { capA = (size_t)B * np * np; d_A.alloc(capA); }
@@ -1022,37 +1403,120 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
                          d_b.p, lu ? 0 : 1);
       DR_HIP(hipGetLastError());
       const int nt = np / NB;
-      for (int k = 0; k < nt; ++k) {
-        const int m = nt - k - 1;
-        if (lu) {
+      if (lu) {
+        for (int k = 0; k < nt; ++k) {
+          const int m = nt - k - 1;
           hipLaunchKernelGGL(k_getrf_panel, dim3(B), dim3(256), 0, s, d_A.p, d_b.p, np, k, d_fail.p);
           if (m > 0) {
             hipLaunchKernelGGL(k_trsm_lu, dim3(B, m), dim3(256), 0, s, d_A.p, np, k);
             hipLaunchKernelGGL(k_gemm_lu_mfma, dim3(B, m * m), dim3(256), 0, s, d_A.p, np, k, m);
           }
-        } else {
-          hipLaunchKernelGGL(k_chol_diag, dim3(B), dim3(256), 0, s, d_A.p, np, k, d_fail.p);
-          if (m > 0) hipLaunchKernelGGL(k_chol_panel, dim3(B, m), dim3(256), 0, s, d_A.p, np, k);
+          DR_HIP(hipGetLastError());
         }
-        DR_HIP(hipGetLastError());
-      }
-      if (lu)
         hipLaunchKernelGGL(k_solve_lu, dim3(B), dim3(256), np * sizeof(double), s, d_A.p, np, d_sd.p, d_b.p,
                            d_fail.p, d_sol.p);
-      else
+      } else {
+        cholesky(d_A.p, B, np);
         hipLaunchKernelGGL(k_solve_chol, dim3(B), dim3(256), np * sizeof(double), s, d_A.p, np, d_sd.p, d_b.p,
                            d_sol.p);
+      }
       DR_HIP(hipGetLastError());
       std::vector<int> fail(B);
       d_fail.down(fail.data(), B, s);
       DR_HIP(hipStreamSynchronize(s));
       if (!lu)
         for (int i = 0; i < B; ++i)
-          if (fail[i]) failed.push_back(bu[i]);
+          if (fail[i]) failed.push_back(uids[first + i]);
     }
     return failed;
   };
-  const std::vector<int> indefinite = solve_all(order, false);
+  std::vector<int> direct, order;
+  (via_inverse ? order : direct).resize(nU);
+  std::iota(order.begin(), order.end(), 0);
+  std::iota(direct.begin(), direct.end(), 0);
+  // Slabs of bounded factor and row memory, the largest factorisations first.
+  auto msize = [&](int u) { return std::min(cnt[urow[u]], nP - cnt[urow[u]]); };
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return msize(a) > msize(b); });
+  for (size_t e0 = 0; e0 < order.size();) {
+    std::vector<ExtDesc> ed;
+    std::vector<FacDesc> fd;
+    std::vector<int> fu;  // unique system of each factorisation
+    long dl = 0, fac = 0;
+    size_t e1 = e0;
+    for (; e1 < order.size(); ++e1) {
+      const int u = order[e1], n = cnt[urow[u]], m = msize(u), np = cdiv(m, NB) * NB;
+      if (e1 > e0 && ((double)(fac + (long)np * np) * 8 > budget || (double)(ed.size() + NB) * ld * 8 > 1.5e9)) break;
+      const bool dir = n < nP - n;
+      if (m > 0) {
+        fd.push_back(FacDesc{m, dir ? -1 : (int)ed.size(), dir ? rp[urow[u]] : dl, fac, usol[u]});
+        fu.push_back(u);
+      }
+      if (!dir) {
+        ed.push_back(ExtDesc{rp[urow[u]], n, m, dl, usol[u]});
+        dl += m;
+      }
+      fac += (long)np * np;
+    }
+    e0 = e1;
+    const int E = (int)ed.size(), nf = (int)fd.size(), rows = cdiv(std::max(E, 1), NB) * NB;
+    const long nz = (long)rows * ld;
+    DBuf<double> R0(nz), R1(nz), R2(nz), R3(nz), d_F(fac);
+    DBuf<ExtDesc> d_ed(E);
+    DBuf<FacDesc> d_fd(nf);
+    DBuf<int> d_dl(dl), d_ef(nf);
+    if (E) d_ed.up(ed.data(), E, s);
+    if (nf) {
+      d_fd.up(fd.data(), nf, s);
+      DR_HIP(hipMemsetAsync(d_ef.p, 0, nf * sizeof(int), s));
+    }
+    const size_t bits = (size_t)((nP + 31) / 32) * 4, ys = (size_t)ld * sizeof(double);
+    auto gemm = [&](const double* F, const double* G, const double* C0, double* C) {
+      hipLaunchKernelGGL(k_gemm_xyt, dim3(ntl, rows / NB), dim3(256), 0, s, F, G, ld, ntl, 0, C0, C);
+      DR_HIP(hipGetLastError());
+    };
+    auto zero = [&](double* p) {
+      hipLaunchKernelGGL(k_zero_f64, dim3(1024), dim3(256), 0, s, nz, p);
+      DR_HIP(hipGetLastError());
+    };
+    // w of right-hand sides F: U = F B, y on the absent offsets, w = U + y B
+    auto solve = [&](const double* F, double* W, int first) {
+      if (E) gemm(F, d_B.p, nullptr, R1.p);
+      if (nf) {
+        hipLaunchKernelGGL(k_solve_all, dim3(nf), dim3(256), ys, s, d_fd.p, d_F.p, ld, d_dl.p, R1.p, R2.p, d_kp.p,
+                           d_sol.p, first);
+        DR_HIP(hipGetLastError());
+      }
+      if (E) gemm(R2.p, d_B.p, R1.p, W);
+    };
+    if (rows > E) zero(R0.p);  // the padding rows of the products
+    zero(R2.p);
+    if (E) {
+      hipLaunchKernelGGL(k_extend, dim3(E), dim3(256), bits, s, d_ed.p, nP, ld, d_pidx.p, d_kp.p, R0.p, d_dl.p);
+      DR_HIP(hipGetLastError());
+    }
+    if (nf) {
+      hipLaunchKernelGGL(k_factor_all, dim3(nf), dim3(256), 0, s, d_fd.p, d_B.p, d_Kd.p, ld, d_dl.p, d_pidx.p, d_F.p,
+                         d_ef.p);
+      DR_HIP(hipGetLastError());
+    }
+    solve(R0.p, R3.p, 1);
+    if (E) {  // refinement: w += solve(k' - w K)
+      hipLaunchKernelGGL(k_clear_absent, dim3(E), dim3(256), 0, s, d_ed.p, ld, d_dl.p, R3.p);
+      DR_HIP(hipGetLastError());
+      gemm(R3.p, d_Kd.p, nullptr, R1.p);
+      hipLaunchKernelGGL(k_residual_ext, dim3(E), dim3(256), 0, s, d_ed.p, ld, d_pidx.p, d_kp.p, R1.p, R0.p);
+      DR_HIP(hipGetLastError());
+      solve(R0.p, R0.p, 0);
+      hipLaunchKernelGGL(k_finish_ext, dim3(E), dim3(256), ys, s, d_ed.p, ld, d_pidx.p, R3.p, R0.p, d_sol.p);
+      DR_HIP(hipGetLastError());
+    }
+    std::vector<int> ef(nf);
+    if (nf) d_ef.down(ef.data(), nf, s);
+    DR_HIP(hipStreamSynchronize(s));
+    for (int i = 0; i < nf; ++i)
+      if (ef[i]) direct.push_back(fu[i]);  // again on its own, and by LU if that fails too
+  }
+  const std::vector<int> indefinite = solve_all(direct, false);
   if (!indefinite.empty()) (void)solve_all(indefinite, true);
   std::vector<int> uidd(n_rows);
   for (int i = 0; i < n_rows; ++i) uidd[i] = uid[i] < 0 ? 0 : uid[i];
