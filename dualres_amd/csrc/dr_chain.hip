@@ -2,7 +2,8 @@
 // fused leapfrog updates, CSR kriging products, float64 energies.
 //
 // State layout in HBM (working precision T):
-//   muA, muB  : half spectra of mu (current, proposal)  [M2][M1][M0/2+1]
+//   muA, muB  : half spectra of mu (current, proposal), [M2][M1][M0/2+1] in
+//               column blocks (Spec, dr_kernels.hpp), like all spectral state
 //   p         : half spectrum of the momentum
 //   miA, miB, pim : imaginary chain (DR_STATE_COMPAT only)
 //   invlam    : 1/lambda on the half spectrum, 0 on Z
@@ -132,6 +133,7 @@ struct ChainBase {
   int M[3] = {0, 0, 0};
   int H0 = 0;
   long N = 0, Nh = 0;
+  long Ns = 0;  // elements of a spectral state array (Spec), Nh and its padding
   int reg[3] = {0, 0, 0};
   long nreg = 0;
   long n_h = 0, n_s = 0;
@@ -291,6 +293,7 @@ struct Chain : public ChainBase {
   }
 
   // ------------------------------------------------------------ launch helpers
+  Spec<T> spec() const { return Spec<T>{M[2], M[1] * H0}; }
   template <typename U>
   const AxisFFT<U>& axis_dev(int a) const {
     if constexpr (std::is_same<U, float>::value) return adf[a];
@@ -332,7 +335,7 @@ struct Chain : public ChainBase {
     DR_REQUIRE(k_in >= 1 && k_in <= ad.M && k_out >= 1 && k_out <= ad.M && NB >= 1 && n_outer >= 1, DR_ELOGIC,
                "line pass: bad extents");
     if (lines_ok(a, pid)) {
-      const LineArgs<T> la{ad.tw, NB, NB * n_outer, k_in, k_out, src, s_so, dst, d_so};
+      const LineArgs<T> la{ad.tw, NB, NB * n_outer, k_in, k_out, src, s_so, dst, d_so, 0};
       if (INV ? lines_inverse(ad.M, la, stream) : lines_forward(ad.M, la, stream)) {
         mark();
         return;
@@ -399,6 +402,7 @@ struct Chain : public ChainBase {
     H0 = M[0] / 2 + 1;
     N = (long)M[0] * M[1] * M[2];
     Nh = (long)H0 * M[1] * M[2];
+    Ns = spec().size();
     tau_sq_inv = 1.0 / cfg.theta[0];  // MultiResParameters.h:256
     for (int a = 0; a < 3; ++a) {
       const int len = M[a];
@@ -423,18 +427,24 @@ struct Chain : public ChainBase {
     sums.alloc(NSLOT);
     part.zero(stream);
     sums.zero(stream);
-    invlam.alloc(Nh);
-    lam.alloc(Nh);
-    muA.alloc(Nh);
-    muB.alloc(Nh);
-    p.alloc(Nh);
+    invlam.alloc(Ns);
+    lam.alloc(Ns);
+    muA.alloc(Ns);
+    muB.alloc(Ns);
+    p.alloc(Ns);
+    invlam.zero(stream);  // the padding stays 0
+    lam.zero(stream);
+    muA.zero(stream);
+    muB.zero(stream);
     p.zero(stream);
     T1.alloc(Nh);
     T2.alloc(Nh);
     if (compat()) {
-      miA.alloc(Nh);
-      miB.alloc(Nh);
-      pim.alloc(Nh);
+      miA.alloc(Ns);
+      miB.alloc(Ns);
+      pim.alloc(Ns);
+      miA.zero(stream);
+      miB.zero(stream);
       pim.zero(stream);
     }
     int r[3];
@@ -464,7 +474,7 @@ struct Chain : public ChainBase {
     xr2c<double>(rows, lb, StoreRowC<double>{{}, s2.p, H0});
     strided<double, false>(1, M[2], H0, M[1], M[1], LoadS<double>{{}, s2.p, (long)M[1] * H0, H0},
                            StoreS<double>{{}, s1.p, (long)M[1] * H0, H0});
-    EpiSpectrum<T> es{lam.p, invlam.p, (long)M[1] * H0, H0, pslot(S_ZCOUNT), 0.0};
+    EpiSpectrum<T> es{lam.p, invlam.p, spec(), H0, pslot(S_ZCOUNT), 0.0};
     strided<double, false>(2, 1, M[1] * H0, M[2], M[2], LoadS<double>{{}, s1.p, 0, (long)M[1] * H0}, es, S_ZCOUNT);
     finalize();
     double h[NSLOT];
@@ -478,8 +488,9 @@ struct Chain : public ChainBase {
   }
 
   void get_lambda(double* out) override {
-    std::vector<double> h(Nh);
-    DR_HIP(hipMemcpyAsync(h.data(), lam.p, Nh * sizeof(double), hipMemcpyDeviceToHost, stream));
+    std::vector<double> h(Ns);
+    const Spec<T> sp = spec();
+    DR_HIP(hipMemcpyAsync(h.data(), lam.p, Ns * sizeof(double), hipMemcpyDeviceToHost, stream));
     DR_HIP(hipStreamSynchronize(stream));
     // expand the Hermitian half spectrum (lambda even and real)
     for (int z = 0; z < M[2]; ++z)
@@ -487,7 +498,7 @@ struct Chain : public ChainBase {
         for (int x = 0; x < M[0]; ++x) {
           int kx = x, ky = y, kz = z;
           if (x >= H0) { kx = M[0] - x; ky = (M[1] - y) % M[1]; kz = (M[2] - z) % M[2]; }
-          out[x + (long)M[0] * (y + (long)M[1] * z)] = h[kx + (long)H0 * (ky + (long)M[1] * kz)];
+          out[x + (long)M[0] * (y + (long)M[1] * z)] = h[sp.at(kz, kx + (long)H0 * ky)];
         }
   }
 
@@ -498,11 +509,11 @@ struct Chain : public ChainBase {
     strided<T, false>(1, M[2], H0, M[1], M[1], LoadS<T>{{}, T2.p, (long)M[1] * H0, H0},
                       StoreS<T>{{}, T1.p, (long)M[1] * H0, H0});
     strided<T, false>(2, 1, M[1] * H0, M[2], M[2], LoadS<T>{{}, T1.p, 0, (long)M[1] * H0},
-                      StoreS<T>{{}, X, 0, (long)M[1] * H0});
+                      StoreSpec<T>{{}, X, spec()});
   }
   // half spectrum X -> full real torus dst, scaled by 1/N
   void c2r_full(const cx<T>* X, T* dst) {
-    strided<T, true>(2, 1, M[1] * H0, M[2], M[2], LoadS<T>{{}, X, 0, (long)M[1] * H0},
+    strided<T, true>(2, 1, M[1] * H0, M[2], M[2], LoadSpec<T>{{}, X, spec()},
                      StoreS<T>{{}, T1.p, 0, (long)M[1] * H0});
     strided<T, true>(1, M[2], H0, M[1], M[1], LoadS<T>{{}, T1.p, (long)M[1] * H0, H0},
                      StoreS<T>{{}, T2.p, (long)M[1] * H0, H0});
@@ -514,7 +525,14 @@ struct Chain : public ChainBase {
     c2r_yx(R);
   }
   // inverse z pass of X into T1 (z < n2)
-  void z_inverse(const cx<T>* X) { line_pass<true>(2, 1, M[1] * H0, M[2], reg[2], X, 0, T1.p, 0); }
+  void z_inverse(const cx<T>* X) {
+    const int NB = M[1] * H0;
+    if (lines_ok(2, -1)) {
+      const LineArgs<T> la{axis_dev<T>(2).tw, NB, NB, M[2], reg[2], X, 0, T1.p, 0, M[2]};
+      if (lines_inverse(M[2], la, stream)) return;
+    }
+    strided<T, true>(2, 1, NB, M[2], reg[2], LoadSpec<T>{{}, X, spec()}, StoreS<T>{{}, T1.p, 0, NB});
+  }
   // forward transform from the image region; Pro is the x-pass prologue,
   // Epi the z-pass epilogue
   template <class Pro, class Epi>
@@ -541,12 +559,11 @@ struct Chain : public ChainBase {
   // the spectral momentum drawn directly (k_momentum_direct), E0 sums to slot
   void momentum_direct(uint64_t stream_id, cx<T>* dst, int slot) {
     DR_REQUIRE(M[0] % 2 == 0 && M[1] % 2 == 0 && M[2] % 2 == 0, DR_ELOGIC, "momentum draw: odd torus size");
-    const long Nh = (long)H0 * M[1] * M[2];
-    DR_REQUIRE(Nh < (1L << 31), DR_ELOGIC, "momentum draw: half spectrum too large for 32-bit indices");
-    const int g = (int)std::min<long>(cdiv(Nh / 2, kThreads), 4096);  // two modes per thread
+    DR_REQUIRE(Ns < (1L << 31), DR_ELOGIC, "momentum draw: half spectrum too large for 32-bit indices");
+    const int g = (int)std::min<long>(cdiv(Ns / 2, kThreads), 4096);  // two modes per thread
     note_blocks(slot, g);
     const double nN = (double)M[0] * M[1] * M[2];
-    hipLaunchKernelGGL(k_momentum_direct<T>, dim3(g), dim3(kThreads), 0, stream, Nh, H0, M[1], M[2], cfg.seed,
+    hipLaunchKernelGGL(k_momentum_direct<T>, dim3(g), dim3(kThreads), 0, stream, Ns, spec(), H0, M[1], M[2], cfg.seed,
                        stream_id, (int)(stream_id & 1), (T)sigma[0], invlam.p, dst, pslot(slot), gsc,
                        (T)std::sqrt(0.5 * nN), (T)std::sqrt(nN));
     DR_HIP(hipGetLastError());
@@ -571,8 +588,8 @@ struct Chain : public ChainBase {
   // ------------------------------------------------------------ init
   void init_mu() {
     // mu = B(F(z) sqrt(lambda) / (10 N)) with z complex normal (:743-759)
-    noise_r2c(2, nullptr, S_TMP, EpiInitMu<T>{{}, muA.p, lam.p, (long)M[1] * H0});
-    if (compat()) noise_r2c(3, nullptr, S_TMP, EpiInitMu<T>{{}, miA.p, lam.p, (long)M[1] * H0});
+    noise_r2c(2, nullptr, S_TMP, EpiInitMu<T>{{}, muA.p, lam.p, spec()});
+    if (compat()) noise_r2c(3, nullptr, S_TMP, EpiInitMu<T>{{}, miA.p, lam.p, spec()});
     stats_valid = false;
   }
 
@@ -1372,7 +1389,7 @@ struct Chain : public ChainBase {
 
   void add_data_to_mu() override {
     DR_REQUIRE(data_set, DR_ELOGIC, "add_data_to_mu: data not set");
-    r2c_region(LoadRowR<T>{{}, Yg.p, reg[0]}, EpiAddTo<T>{{}, muA.p, (long)M[1] * H0}, -1, -1);
+    r2c_region(LoadRowR<T>{{}, Yg.p, reg[0]}, EpiAddTo<T>{{}, muA.p, spec()}, -1, -1);
     stats_valid = false;
   }
 
@@ -1568,7 +1585,7 @@ struct Chain : public ChainBase {
         rec = 0;
         mark();
       }
-      MidLeapfrog<T> mid{s == 0 ? muA.p : muB.p, muB.p, p.p, invlam.p, sk, (T)((s == 0 ? 0.5 : 1.0) * eps),
+      MidLeapfrog<T> mid{s == 0 ? muA.p : muB.p, muB.p, p.p, invlam.p, spec(), (T)((s == 0 ? 0.5 : 1.0) * eps),
                          (T)eps, (T)sigma[0], H0, s == 0 ? 1 : 0, pslot(S_PRIOR_A), 0.0, gsc, s == 0 ? 0 : 1};
       zfused(mid, s == 0 ? S_PRIOR_A : -1);
       likelihood(RB.p, last ? S_SSEH_B : -1, last ? S_SSES_B : -1, last);
@@ -1579,7 +1596,7 @@ struct Chain : public ChainBase {
       if (prof && L >= 2 && s == L - 1) DR_HIP(hipEventRecord(ev[1], stream));
     }
     // final half kick at B with the energies of the end point
-    EpiMomentum<T> em{muB.p, p.p, invlam.p, sk, (T)(0.5 * eps), (T)sigma[0], H0, nullptr, nullptr, 1, part.p,
+    EpiMomentum<T> em{muB.p, p.p, invlam.p, spec(), (T)(0.5 * eps), (T)sigma[0], H0, nullptr, nullptr, 1, part.p,
                       pstride, S_PRIOR_B, S_TMP, S_KIN_B, S_TMP, 0.0, 0.0, 0.0, 0.0, gsc};
     const int zb = zgrid();
     note_blocks(S_PRIOR_B, zb);
@@ -1588,11 +1605,11 @@ struct Chain : public ChainBase {
     strided<T, false>(2, 1, M[1] * H0, reg[2], M[2], LoadS<T>{{}, T1.p, 0, sk}, em);
     if (compat()) {
       // imaginary chain: all L steps per mode in one pass
-      const int g = (int)std::min<long>(cdiv(Nh, kThreads), 4096);
+      const int g = (int)std::min<long>(cdiv(Ns, kThreads), 4096);
       note_blocks(S_PRIORI_A, g);
       note_blocks(S_PRIORI_B, g);
       note_blocks(S_KINI_B, g);
-      hipLaunchKernelGGL(k_imag_leapfrog<T>, dim3(g), dim3(kThreads), 0, stream, Nh, H0, miA.p, miB.p, pim.p,
+      hipLaunchKernelGGL(k_imag_leapfrog<T>, dim3(g), dim3(kThreads), 0, stream, Ns, spec(), H0, miA.p, miB.p, pim.p,
                          invlam.p, (T)eps, (T)(0.5 * eps), (T)eps, (T)sigma[0], L, pslot(S_PRIORI_A),
                          pslot(S_PRIORI_B), pslot(S_KINI_B), gsc);
       DR_HIP(hipGetLastError());
@@ -1609,14 +1626,13 @@ struct Chain : public ChainBase {
   // momentum draw and leapfrog of one HMC iteration, then the energy sums
   // (MultiResParameters.h:680-705); normals injected when zr is given
   void device_iteration(double eps, int L, uint64_t it, const double* zr, const double* zi) {
-    const long sk = (long)M[1] * H0;
     clear_slots();
     // injected real-space normals go through the transforms; the product
     // path draws the spectral momentum directly
     if (zr) {
       upload_real(zr, zbuf);
       noise_r2c(4 * it + 0, zbuf.p, S_E0,
-                EpiNoiseMomentum<T>{p.p, invlam.p, sk, (T)sigma[0], gsc, H0, pslot(S_E0), 0.0});
+                EpiNoiseMomentum<T>{p.p, invlam.p, spec(), (T)sigma[0], gsc, H0, pslot(S_E0), 0.0});
     } else {
       momentum_direct(4 * it + 0, p.p, S_E0);
     }
@@ -1624,7 +1640,7 @@ struct Chain : public ChainBase {
       if (zr) {
         upload_real(zi, zbuf);
         noise_r2c(4 * it + 1, zbuf.p, S_E0I,
-                  EpiNoiseMomentum<T>{pim.p, invlam.p, sk, (T)sigma[0], gsc, H0, pslot(S_E0I), 0.0});
+                  EpiNoiseMomentum<T>{pim.p, invlam.p, spec(), (T)sigma[0], gsc, H0, pslot(S_E0I), 0.0});
       } else {
         momentum_direct(4 * it + 1, pim.p, S_E0I);
       }
@@ -1692,8 +1708,8 @@ struct Chain : public ChainBase {
 
   // ------------------------------------------------------------ captured iterations
   void accept_copy(hipStream_t s) {
-    DR_HIP(hipMemcpyAsync(muA.p, muB.p, Nh * sizeof(cx<T>), hipMemcpyDeviceToDevice, s));
-    if (compat()) DR_HIP(hipMemcpyAsync(miA.p, miB.p, Nh * sizeof(cx<T>), hipMemcpyDeviceToDevice, s));
+    DR_HIP(hipMemcpyAsync(muA.p, muB.p, Ns * sizeof(cx<T>), hipMemcpyDeviceToDevice, s));
+    if (compat()) DR_HIP(hipMemcpyAsync(miA.p, miB.p, Ns * sizeof(cx<T>), hipMemcpyDeviceToDevice, s));
     DR_HIP(hipMemcpyAsync(RA.p, RB.p, (nreg + 4) * sizeof(T), hipMemcpyDeviceToDevice, s));
   }
   // forget captured graphs when buffers move; a batch compares layout_gen
@@ -1922,9 +1938,9 @@ struct Chain : public ChainBase {
   }
 
   void quad(const cx<T>* X, int slot, T sig) {
-    const int g = (int)std::min<long>(cdiv(Nh, kThreads), 2048);
+    const int g = (int)std::min<long>(cdiv(Ns, kThreads), 2048);
     note_blocks(slot, g);
-    hipLaunchKernelGGL(k_quad<T>, dim3(g), dim3(kThreads), 0, stream, Nh, H0, X, invlam.p, sig, pslot(slot));
+    hipLaunchKernelGGL(k_quad<T>, dim3(g), dim3(kThreads), 0, stream, Ns, spec(), H0, X, invlam.p, sig, pslot(slot));
     DR_HIP(hipGetLastError());
   }
 
@@ -1956,13 +1972,13 @@ struct Chain : public ChainBase {
   void set_tau_sq_inv(double t) override {
     DR_REQUIRE(t > 0.0 && std::isfinite(t), DR_EDOMAIN, "tau^-2 must be positive and finite");
     if (!invlam0.p) {
-      invlam0.alloc(Nh);
-      lam0.alloc(Nh);
-      DR_HIP(hipMemcpyAsync(invlam0.p, invlam.p, Nh * sizeof(T), hipMemcpyDeviceToDevice, stream));
-      DR_HIP(hipMemcpyAsync(lam0.p, lam.p, Nh * sizeof(double), hipMemcpyDeviceToDevice, stream));
+      invlam0.alloc(Ns);
+      lam0.alloc(Ns);
+      DR_HIP(hipMemcpyAsync(invlam0.p, invlam.p, Ns * sizeof(T), hipMemcpyDeviceToDevice, stream));
+      DR_HIP(hipMemcpyAsync(lam0.p, lam.p, Ns * sizeof(double), hipMemcpyDeviceToDevice, stream));
     }
     const double t0 = 1.0 / cfg.theta[0];
-    hipLaunchKernelGGL(k_rescale_spectrum<T>, dim3(cdiv(Nh, kThreads)), dim3(kThreads), 0, stream, (long)Nh,
+    hipLaunchKernelGGL(k_rescale_spectrum<T>, dim3(cdiv(Ns, kThreads)), dim3(kThreads), 0, stream, Ns,
                        invlam0.p, lam0.p, invlam.p, lam.p, (T)(t0 / t), t / t0);
     DR_HIP(hipGetLastError());
     tau_sq_inv = t;
@@ -2024,16 +2040,15 @@ struct Chain : public ChainBase {
   void gradient(double* gr, double* gi) override {
     DR_REQUIRE(data_set, DR_ELOGIC, "gradient: data not set");
     if (Rf.n != (size_t)N) Rf.alloc(N);
-    const long sk = (long)M[1] * H0;
     c2r_region(muA.p, RA.p);
     w_products(RA.p, -1);
-    r2c_region(residual(RA.p, -1), EpiGrad<T>{{}, muA.p, muB.p, invlam.p, sk}, -1, -1);
+    r2c_region(residual(RA.p, -1), EpiGrad<T>{{}, muA.p, muB.p, invlam.p, spec()}, -1, -1);
     c2r_full(muB.p, Rf.p);
     download_real(Rf, gr);
     if (gi) {
       if (compat()) {
-        DR_HIP(hipMemcpyAsync(muB.p, miA.p, Nh * sizeof(cx<T>), hipMemcpyDeviceToDevice, stream));
-        hipLaunchKernelGGL(k_scale_spec<T>, dim3(cdiv(Nh, kThreads)), dim3(kThreads), 0, stream, Nh, muB.p, invlam.p,
+        DR_HIP(hipMemcpyAsync(muB.p, miA.p, Ns * sizeof(cx<T>), hipMemcpyDeviceToDevice, stream));
+        hipLaunchKernelGGL(k_scale_spec<T>, dim3(cdiv(Ns, kThreads)), dim3(kThreads), 0, stream, Ns, muB.p, invlam.p,
                            (T)-1);
         DR_HIP(hipGetLastError());
         c2r_full(muB.p, Rf.p);
@@ -2120,8 +2135,9 @@ int dr_estimate_bytes(const dr_config* cfg, const int32_t* ijk, int64_t n_h, int
     const int64_t s = cfg->precision == DR_FP64 ? 8 : 4, cb = 2 * s;
     const int64_t H0 = M[0] / 2 + 1, Nh = H0 * M[1] * M[2];
     const int64_t nreg = (int64_t)(mx[0] + 1) * (mx[1] + 1) * (mx[2] + 1);
-    int64_t b = Nh * (5 * cb + s + 8);                                   // mu A/B, p, T1, T2, 1/lambda, lambda
-    if (cfg->state_mode == DR_STATE_COMPAT) b += 3 * Nh * cb;            // imaginary chain
+    const int64_t Ns = (H0 * M[1] + 15) / 16 * 16 * M[2];                // spectral arrays, whole column blocks
+    int64_t b = Ns * (3 * cb + s + 8) + 2 * Nh * cb;                     // mu A/B, p, 1/lambda, lambda; T1, T2
+    if (cfg->state_mode == DR_STATE_COMPAT) b += 3 * Ns * cb;            // imaginary chain
     int64_t ps = std::max<int64_t>({1024, Nh / 8 + 1, (int64_t)M[1] * M[2] + 1, (int64_t)M[1] * H0 + 1});
     if (n_s > 0) ps = std::max<int64_t>(ps, (n_s + 3) / 4 + n_s + 2);
     b += 16 * ps * 8;                                                    // reduction partials

@@ -2,7 +2,7 @@
 // of the gradient: CSR W.mu, W^T v, reductions.
 //
 // Spectral arrays hold the half spectrum S[kz][ky][kx], kx in [0, M0/2],
-// of real torus fields.  invlam[k] = 1/lambda_k for lambda_k > 0 and 0 on
+// of real torus fields; the chain's state keeps its columns in blocks (Spec).  invlam[k] = 1/lambda_k for lambda_k > 0 and 0 on
 // the low-rank set Z (Re lambda <= 0), which implements every "zero Z" of
 // the reference (MultiResParameters.h:309-319) with a single array.
 #pragma once
@@ -35,6 +35,25 @@ __device__ __forceinline__ void red_write(double v, double* red, double* part, i
   if (threadIdx.x == 0) part[blk] = s;
 }
 
+// Layout of the spectral state (mu, p, 1 / lambda, lambda): the columns
+// c = kx + H0 ky of the z lines in blocks of C, each block [kz][C], so that
+// the z pass streams a workgroup's state from one contiguous piece.  As rows
+// of 128 bytes, M1 H0 elements apart, the same bytes came at 4.4 to 4.8 TB/s
+// (z pass at 256x512x256 in float64 330 us, 240 us in blocks; at 256x320x256
+// in float32 97 and 84).  C columns are 128 bytes of the state.  Columns that
+// pad the last block hold 0 everywhere.
+template <typename T> struct Spec {
+  static constexpr int L = sizeof(T) == 4 ? 4 : 3, C = 1 << L;
+  int M2, NB;  // kz rows, columns
+  __host__ __device__ __forceinline__ long at(long k, long c) const { return ((c >> L) * M2 + k) * C + (c & (C - 1)); }
+  // column of element i, NB or more in the padding
+  __host__ __device__ __forceinline__ unsigned col(unsigned long i) const {
+    return ((unsigned)(i >> L) / (unsigned)M2) * C + (unsigned)(i & (C - 1));
+  }
+  __host__ __device__ __forceinline__ unsigned row(unsigned long i) const { return (unsigned)(i >> L) % (unsigned)M2; }
+  __host__ long size() const { return (long)((NB + C - 1) / C) * C * M2; }
+};
+
 // ---------------------------------------------------------------- strided functors
 template <typename T> struct LoadS : NoRed {
   const cx<T>* src; long so, sk;
@@ -45,27 +64,21 @@ template <typename T> struct StoreS : NoRed {
   __device__ __forceinline__ void store(int o, int k, int b, cx<T> v) const { dst[o * so + (long)k * sk + b] = v; }
 };
 
-// position update mu += eps * M^{-1} p fused into the first inverse pass
-// (MultiResParameters.h:693-698): M^{-1} = 1 / (1/lambda + sigma_h^-2), 0 on Z.
-template <typename T> struct LoadPosUpdate : NoRed {
-  const cx<T>* src; cx<T>* dst; const cx<T>* p; const T* invlam; long sk; T eps; T sig;
-  const cx<T>* srci; cx<T>* dsti; const cx<T>* pim;  // imaginary chain (may be null)
-  __device__ __forceinline__ cx<T> load(int, int k, int b) const {
-    const long i = (long)k * sk + b;
-    const T il = invlam[i];
-    const T c = il > (T)0 ? eps / (il + sig) : (T)0;
-    const cx<T> m = src[i] + p[i] * c;
-    dst[i] = m;
-    if (dsti) dsti[i] = srci[i] + pim[i] * c;
-    return m;
-  }
+// columns of the spectral state
+template <typename T> struct LoadSpec : NoRed {
+  const cx<T>* src; Spec<T> sp;
+  __device__ __forceinline__ cx<T> load(int, int k, int b) const { return src[sp.at(k, b)]; }
+};
+template <typename T> struct StoreSpec : NoRed {
+  cx<T>* dst; Spec<T> sp;
+  __device__ __forceinline__ void store(int, int k, int b, cx<T> v) const { dst[sp.at(k, b)] = v; }
 };
 
 // momentum update p += coef * (F(S r) - mu/lambda) fused into the last
 // forward pass (MultiResParameters.h:690,699 with _compute_gradient :349-374);
 // optional reductions of the prior and kinetic energies (Parseval).
 template <typename T> struct EpiMomentum {
-  const cx<T>* X; cx<T>* p; const T* invlam; long sk; T coef; T sig; int H0;
+  const cx<T>* X; cx<T>* p; const T* invlam; Spec<T> sp; T coef; T sig; int H0;
   const cx<T>* Xi; cx<T>* pim;
   int do_red; double* part; long pstride; int s_prior, s_priori, s_kin, s_kini;
   double a0, a1, a2, a3;
@@ -80,7 +93,7 @@ template <typename T> struct EpiMomentum {
   // state before updating them)
   struct State { T il; cx<T> x, p, xi, pi; };
   __device__ __forceinline__ State fetch(int, int k, int b) const {
-    const long i = (long)k * sk + b;
+    const long i = sp.at(k, b);
     State s{invlam[i], X[i], p[i], mk<T>(0, 0), mk<T>(0, 0)};
     if (pim) {
       s.xi = Xi[i];
@@ -90,7 +103,7 @@ template <typename T> struct EpiMomentum {
   }
   __device__ __forceinline__ void store(int o, int k, int b, cx<T> v) { store(o, k, b, v, fetch(o, k, b)); }
   __device__ __forceinline__ void store(int, int k, int b, cx<T> v, const State& s) {
-    const long i = (long)k * sk + b;
+    const long i = sp.at(k, b);
     const T il = s.il;
     const cx<T> x = s.x;
     const cx<T> pn = s.p + (v - x * il) * coef;
@@ -141,7 +154,7 @@ __device__ __forceinline__ void nt_st(cx<T>* q, cx<T> v) {
   __builtin_nontemporal_store(v2{v.x, v.y}, reinterpret_cast<v2*>(q));
 }
 template <typename T> struct MidLeapfrog {
-  const cx<T>* X; cx<T>* Xd; cx<T>* p; const T* invlam; long sk; T coef; T eps; T sig; int H0;
+  const cx<T>* X; cx<T>* Xd; cx<T>* p; const T* invlam; Spec<T> sp; T coef; T eps; T sig; int H0;
   int do_red; double* part; double a0;
   const StepScalars<T>* sc; int coef_full;  // coef = full (1) or half (0) step
   __device__ __forceinline__ void bind() {
@@ -171,9 +184,9 @@ template <typename T> struct MidLeapfrog {
     }
     return m;
   }
-  __device__ __forceinline__ State fetch(int k, int b) const { return fetch_at((long)k * sk + b); }
+  __device__ __forceinline__ State fetch(int k, int b) const { return fetch_at(sp.at(k, b)); }
   __device__ __forceinline__ cx<T> apply(int k, int b, cx<T> v, const State& s) {
-    return apply_at((long)k * sk + b, b, v, s, true);
+    return apply_at(sp.at(k, b), b, v, s, true);
   }
   __device__ __forceinline__ cx<T> apply(int k, int b, cx<T> v) { return apply(k, b, v, fetch(k, b)); }
   __device__ __forceinline__ void finish(double* red, int blk) {
@@ -188,7 +201,7 @@ template <typename T> struct MidLeapfrog {
 // and after and its final kinetic energy.
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
-k_imag_leapfrog(long Nh, int H0, const cx<T>* __restrict__ muA, cx<T>* __restrict__ muB, cx<T>* __restrict__ p,
+k_imag_leapfrog(long n, Spec<T> sp, int H0, const cx<T>* __restrict__ muA, cx<T>* __restrict__ muB, cx<T>* __restrict__ p,
                 const T* __restrict__ invlam, T eps, T half_coef, T full_coef, T sig, int L, double* partA,
                 double* partB, double* partK, const StepScalars<T>* sc) {
   __shared__ double red[kThreads];
@@ -199,12 +212,12 @@ k_imag_leapfrog(long Nh, int H0, const cx<T>* __restrict__ muA, cx<T>* __restric
     sig = sc->sig0;
   }
   double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-  for (long i = (long)blockIdx.x * kThreads + threadIdx.x; i < Nh; i += (long)gridDim.x * kThreads) {
+  for (long i = (long)blockIdx.x * kThreads + threadIdx.x; i < n; i += (long)gridDim.x * kThreads) {
     const T il = invlam[i];
     const T c = il > (T)0 ? eps / (il + sig) : (T)0;
     cx<T> m = muA[i];
     cx<T> q = p[i];
-    const double w = herm_w((int)(i % H0), H0);
+    const double w = herm_w((int)(sp.col(i) % (unsigned)H0), H0);
     a0 += w * (double)il * ((double)m.x * m.x + (double)m.y * m.y);
     q = q - m * (il * half_coef);
     for (int s = 0; s < L; ++s) {
@@ -224,9 +237,9 @@ k_imag_leapfrog(long Nh, int H0, const cx<T>* __restrict__ muA, cx<T>* __restric
 
 // gradient in the spectral domain: G = F(S r) - X/lambda
 template <typename T> struct EpiGrad : NoRed {
-  const cx<T>* X; cx<T>* G; const T* invlam; long sk;
+  const cx<T>* X; cx<T>* G; const T* invlam; Spec<T> sp;
   __device__ __forceinline__ void store(int, int k, int b, cx<T> v) const {
-    const long i = (long)k * sk + b;
+    const long i = sp.at(k, b);
     G[i] = v - X[i] * invlam[i];
   }
 };
@@ -241,19 +254,19 @@ template <typename T> struct EpiGrad : NoRed {
 // ulp, and that difference between E0 and the end point's kinetic energy
 // would shift every accept ratio (by about exp(2.7) at the 1 mm workload).
 template <typename T> struct EpiNoiseMomentum {
-  cx<T>* p; const T* invlam; long sk; T sig;
+  cx<T>* p; const T* invlam; Spec<T> sp; T sig;
   const StepScalars<T>* sc;
   int H0; double* part; double acc;
   __device__ __forceinline__ void bind() {
     if (sc) sig = sc->sig0;
   }
   struct State { T il; };
-  __device__ __forceinline__ State fetch(int, int k, int b) const { return State{invlam[(long)k * sk + b]}; }
+  __device__ __forceinline__ State fetch(int, int k, int b) const { return State{invlam[sp.at(k, b)]}; }
   __device__ __forceinline__ void store(int o, int k, int b, cx<T> v) { store(o, k, b, v, fetch(o, k, b)); }
   // sqrt in T: the correctly rounded float square root equals the float
   // rounding of the double one
   __device__ __forceinline__ void store(int, int k, int b, cx<T> v, const State& s) {
-    const long i = (long)k * sk + b;
+    const long i = sp.at(k, b);
     const T il = s.il;
     const cx<T> pn = il > (T)0 ? v * sqrt(il + sig) : mk<T>(0, 0);
     p[i] = pn;
@@ -280,7 +293,9 @@ template <typename T> struct EpiNoiseMomentum {
 // (53-bit uniforms from its four words).  Float32: from block q / 2, words
 // (a, c) for even q and (b, d) for odd q, so a thread's two consecutive modes
 // share one block.  E0 is summed as EpiNoiseMomentum sums it.  Even M0, M1,
-// M2 (Nh is even, below 2^31: the index arithmetic is 32-bit).
+// M2 (two neighbouring columns, a thread's pair, then lie in one block of the
+// layout and are both columns or both padding, which is left at 0; below 2^31
+// elements: the index arithmetic is 32-bit).
 struct ModeKey {
   uint32_t key, kx;
   bool self, cj;
@@ -300,7 +315,7 @@ __device__ __forceinline__ ModeKey mode_key(uint32_t i, uint32_t H0, uint32_t M1
 
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
-k_momentum_direct(long Nh, int H0, int M1, int M2, uint64_t seed, uint64_t stream, int which, T sig,
+k_momentum_direct(long n, Spec<T> sp, int H0, int M1, int M2, uint64_t seed, uint64_t stream, int which, T sig,
                   const T* __restrict__ invlam, cx<T>* __restrict__ p, double* part, const StepScalars<T>* sc,
                   T sd_pair, T sd_self) {
   __shared__ double red[kThreads];
@@ -309,11 +324,14 @@ k_momentum_direct(long Nh, int H0, int M1, int M2, uint64_t seed, uint64_t strea
     sig = sc->sig0;
   }
   double acc = 0.0;
-  for (uint32_t t = blockIdx.x * kThreads + threadIdx.x; 2 * (long)t < Nh; t += gridDim.x * kThreads) {
+  for (uint32_t t = blockIdx.x * kThreads + threadIdx.x; 2 * (long)t < n; t += gridDim.x * kThreads) {
+    const uint32_t c0 = sp.col(2 * t);
+    if (c0 >= (uint32_t)sp.NB) continue;
+    const uint32_t i0 = sp.row(2 * t) * (uint32_t)sp.NB + c0;  // mode index
     ModeKey m[2];
     T a[2], b[2];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) m[u] = mode_key(2 * t + u, (uint32_t)H0, (uint32_t)M1, (uint32_t)M2);
+    for (int u = 0; u < 2; ++u) m[u] = mode_key(i0 + u, (uint32_t)H0, (uint32_t)M1, (uint32_t)M2);
     if constexpr (sizeof(T) == 4) {
       const u4 r0 = philox_block(seed, stream, (uint64_t)(m[0].key >> 1));
       const u4 r1 = (m[1].key >> 1) == (m[0].key >> 1) ? r0 : philox_block(seed, stream, (uint64_t)(m[1].key >> 1));
@@ -341,18 +359,18 @@ k_momentum_direct(long Nh, int H0, int M1, int M2, uint64_t seed, uint64_t strea
 
 // initial state mu = sqrt(lambda) F(z) / 10, 0 on Z (MultiResParameters.h:752-755)
 template <typename T> struct EpiInitMu : NoRed {
-  cx<T>* X; const double* lam; long sk;
+  cx<T>* X; const double* lam; Spec<T> sp;
   __device__ __forceinline__ void store(int, int k, int b, cx<T> v) const {
-    const long i = (long)k * sk + b;
+    const long i = sp.at(k, b);
     const double l = lam[i];
     X[i] = l > 0.0 ? v * (T)(sqrt(l) / 10.0) : mk<T>(0, 0);
   }
 };
 
 template <typename T> struct EpiAddTo : NoRed {
-  cx<T>* X; long sk;
+  cx<T>* X; Spec<T> sp;
   __device__ __forceinline__ void store(int, int k, int b, cx<T> v) const {
-    const long i = (long)k * sk + b;
+    const long i = sp.at(k, b);
     X[i] = X[i] + v;
   }
 };
@@ -360,9 +378,9 @@ template <typename T> struct EpiAddTo : NoRed {
 // eigenvalues: lambda = Re F(c); invlam for the working precision; weighted
 // count of Re lambda <= 0 (MultiResParameters.h:253-262)
 template <typename T> struct EpiSpectrum {
-  double* lam; T* invlam; long sk; int H0; double* part; double acc;
+  double* lam; T* invlam; Spec<T> sp; int H0; double* part; double acc;
   __device__ __forceinline__ void store(int, int k, int b, cx<double> v) {
-    const long i = (long)k * sk + b;
+    const long i = sp.at(k, b);
     lam[i] = v.x;
     invlam[i] = v.x > 0.0 ? (T)(1.0 / v.x) : (T)0;
     if (!(v.x > 0.0)) acc += herm_w(b % H0, H0);
@@ -981,15 +999,15 @@ k_sum_acc(long n, const T* __restrict__ v, const unsigned long long* __restrict_
 // 1/(invlam + sig) (kinetic); sig < 0 selects the prior form.
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
-k_quad(long Nh, int H0, const cx<T>* __restrict__ X, const T* __restrict__ invlam, T sig, double* part) {
+k_quad(long n, Spec<T> sp, int H0, const cx<T>* __restrict__ X, const T* __restrict__ invlam, T sig, double* part) {
   __shared__ double red[kThreads];
   double acc = 0.0;
-  for (long i = (long)blockIdx.x * kThreads + threadIdx.x; i < Nh; i += (long)gridDim.x * kThreads) {
+  for (long i = (long)blockIdx.x * kThreads + threadIdx.x; i < n; i += (long)gridDim.x * kThreads) {
     const T il = invlam[i];
     double a = (double)il;
     if (sig >= (T)0) a = il > (T)0 ? 1.0 / (double)(il + sig) : 0.0;
     const cx<T> x = X[i];
-    acc += herm_w((int)(i % H0), H0) * a * ((double)x.x * x.x + (double)x.y * x.y);
+    acc += herm_w((int)(sp.col(i) % (unsigned)H0), H0) * a * ((double)x.x * x.x + (double)x.y * x.y);
   }
   red_write(acc, red, part, blockIdx.x);
 }

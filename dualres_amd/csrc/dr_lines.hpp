@@ -185,10 +185,12 @@ __device__ __forceinline__ double line_sum(double x, double* sh) {
 // nothing else, so small radices (three stages, more threads per line, 30 to
 // 60 registers) hide more latency: at 1 mm the inverse y pass (320) took 19.3
 // us with 8 8 5 against 23.4 with 20 16, at 1.5 mm (200) 9.9 with 8 5 5
-// against 12.8 with 20 10.  The z pass also holds the state of its modes and
-// gains from fewer exchanges: 96 us with 16 16 against 109 with 8 8 4.
+// against 12.8 with 20 10.  The z pass also holds the state of its modes: in
+// float32 it gains from fewer exchanges (84 us with 16 16 at 256x320x256, 96
+// with 8 8 4), in float64 from fewer registers (240 us with 8 8 4 at
+// 256x512x256, 280 with 16 16).
 constexpr int kCapStrided = 10;
-template <typename T> constexpr int line_cap() { return sizeof(T) == 4 ? 20 : 16; }
+template <typename T> constexpr int line_cap() { return sizeof(T) == 4 ? 20 : 10; }
 // columns per workgroup: runs of 128 bytes per row, more where lines are
 // short, fewer where 16 lines would need over 1024 threads
 template <typename T> constexpr int line_cols(int nj) { return nj < 16 || (sizeof(T) == 4 && nj <= 64) ? 16 : 8; }
@@ -213,6 +215,7 @@ template <typename T> struct LineArgs {
   long s_so;
   cx<T>* dst;
   long d_so;
+  int spec;  // rows M2 of a source in the spectral state's layout (one outer index), or 0
 };
 template <typename T, bool INV, int M>
 __global__ void __launch_bounds__((StridedShape<T, M>::NT))
@@ -225,7 +228,9 @@ k_lines(LineArgs<T> a) {
   const int c = xcd_tile(blockIdx.x, gridDim.x) * TB + b;
   const bool in = c < a.ncol;
   const int cc = in ? c : a.ncol - 1, o = cc / a.nb, bc = cc - o * a.nb;
-  const cx<T>* s = a.src + (o * a.s_so + bc);
+  // element k of the column at s + k * sk
+  const cx<T>* s = a.src + (a.spec ? Spec<T>{a.spec, a.nb}.at(0, bc) : o * a.s_so + bc);
+  const int sk = a.spec ? Spec<T>::C : a.nb;
   cx<T> v[Plan::rmax];
   if (j < B1) {
 #pragma unroll
@@ -233,7 +238,7 @@ k_lines(LineArgs<T> a) {
       v[r] = mk<T>(0, 0);
       if (r * B1 < a.k_in) {  // uniform; rows past the input are zero
         const int k = j + r * B1;
-        const cx<T> x = s[(unsigned)(min(k, a.k_in - 1) * a.nb)];
+        const cx<T> x = s[(unsigned)(min(k, a.k_in - 1) * sk)];
         v[r].x = k < a.k_in ? x.x : (T)0;
         v[r].y = k < a.k_in ? x.y : (T)0;
       }
@@ -287,24 +292,27 @@ k_zlines(const cx<T>* tw, int nb, int n_in, int n_out, cx<T>* T1, MidLeapfrog<T>
       }
     }
   }
+  // mode k of the column in the state's layout
+  const unsigned s0 = (unsigned)Spec<T>{M, nb}.at(0, cc);
+  auto si = [&](int k) { return s0 + (unsigned)(k * Spec<T>::C); };
   typename MidLeapfrog<T>::State st[NP];
 #pragma unroll
-  for (int r = 0; r < NP; ++r) st[r] = mid.fetch_at((unsigned)((j + r * BL) * nb + cc));
+  for (int r = 0; r < NP; ++r) st[r] = mid.fetch_at(si(j + r * BL));
   auto at = [&](int i) { return &buf[i * TB + b]; };
   line_fft<T, Plan, M, false, false, 1>(v, j, tw, at, false);
   // every thread owns RL modes (BL is the widest stage); a tail column works
   // on the last one's values and stores nothing
 #pragma unroll
-  for (int r = 0; r < NP; ++r) v[r] = mid.apply_at((unsigned)((j + r * BL) * nb + cc), cc, v[r], st[r], in);
+  for (int r = 0; r < NP; ++r) v[r] = mid.apply_at(si(j + r * BL), cc, v[r], st[r], in);
 #pragma unroll
   for (int r0 = NP; r0 < RL; r0 += 4) {
     typename MidLeapfrog<T>::State sr[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      if (r0 + u < RL) sr[u] = mid.fetch_at((unsigned)((j + (r0 + u) * BL) * nb + cc));
+      if (r0 + u < RL) sr[u] = mid.fetch_at(si(j + (r0 + u) * BL));
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      if (r0 + u < RL) v[r0 + u] = mid.apply_at((unsigned)((j + (r0 + u) * BL) * nb + cc), cc, v[r0 + u], sr[u], in);
+      if (r0 + u < RL) v[r0 + u] = mid.apply_at(si(j + (r0 + u) * BL), cc, v[r0 + u], sr[u], in);
   }
   line_fft<T, Plan, M, true, true, 1>(v, j, tw, at, true);
   if (j < B1 && in) {
@@ -328,7 +336,7 @@ k_zlines(const cx<T>* tw, int nb, int n_in, int n_out, cx<T>* T1, MidLeapfrog<T>
 // read twice (X[k] and X[Mh - k] meet in Z[k] and Z[Mh - k]), the second time
 // from the cache, in place of an exchange.
 template <typename T, int Mh> struct RowShape {
-  using Plan = LinePlan<Mh, sizeof(T) == 4 ? 20 : 10>;
+  using Plan = LinePlan<Mh, line_cap<T>()>;
   static constexpr int RW = Plan::nj >= 64 ? 1 : 64 / Plan::nj, NT = RW * Plan::nj;
   static constexpr int R1 = Plan::P.r[0];
   // a pad slot after every R1 elements where R1 is even: the first stage
