@@ -229,6 +229,9 @@ struct Chain : public ChainBase {
   DevBuf<double> sm1, sm2, sma;
   DevBuf<unsigned long long> smax;
   int64_t nsum = 0;
+  // voxels past the region and lattice points past the lattice grid that vector
+  // loads of a line's tail may touch, kept 0
+  static constexpr int kPadR = 32, kPadL = 32;
   // stencil + boundary W (see build_stencil)
   struct WStencil {
     DevBuf<int> irow, ibase, ilidx, sub_start, sub_ldo, tiles, mpar, wstart, woff;
@@ -236,6 +239,11 @@ struct Chain : public ChainBase {
     DevBuf<int> brow, brp, bbase, tbase, tg, trp, frow, frp, fcol, tfp, tfidx;
     DevBuf<uint16_t> bd, td;
     DevBuf<T> bw, tw, Vc, fw, tfw, Vf;
+    // interior products by lines along x (lattice step 1..4; 0: the window
+    // table of W mu, sxm, and the voxel tiles of W^T v, sx)
+    int sx = 0, sxm = 0, nc = 0, mc = 0, n_mitem = 0, n_mline = 0, n_titem = 0;
+    DevBuf<int> lm_base, lm_lidx, lm_row, lm_off, lt_vox, lt_x0, lt_vl, lt_cls, lt_start, lt_off;
+    DevBuf<T> lm_w, lt_w;
     int n_int = 0, nD = 0, n_bnd = 0, n_touch = 0, n_far = 0, n_mslot = 0, ncw = 0;
     // interior W^T v tiles: voxel tile dims, LDS box dims, lattice c + sg Z^3,
     // smallest lattice offset, lattice grid box (lo, lv)
@@ -601,8 +609,8 @@ struct Chain : public ChainBase {
     if (r[0] == reg[0] && r[1] == reg[1] && r[2] == reg[2]) return;
     for (int a = 0; a < 3; ++a) reg[a] = r[a];
     nreg = (long)reg[0] * reg[1] * reg[2];
-    RA.alloc(nreg + 4);  // + 4: the aligned 4-voxel windows of W mu may end past the region
-    RB.alloc(nreg + 4);
+    RA.alloc(nreg + kPadR);  // the vector loads of W mu may end past the region
+    RB.alloc(nreg + kPadR);
     RA.zero(stream);
     RB.zero(stream);
     Yg.alloc(nreg);
@@ -983,6 +991,117 @@ struct Chain : public ChainBase {
     std::vector<int32_t> sub_ldo(nD);
     for (int e = 0; e < nD; ++e)
       sub_ldo[e] = (int32_t)(sub_o[3 * e] + LT[0] * (sub_o[3 * e + 1] + LT[1] * sub_o[3 * e + 2]));
+    // 3b. the interior products by stencil lines (wmu_line_block,
+    //     wtv_line_block): the stencil's runs along x, for a lattice step of 1
+    //     to 4 and rows that mostly have their neighbours along x (an item
+    //     works on 4 of them; below 2 present per item the window table does
+    //     less)
+    struct Lines {
+      std::vector<int32_t> off;
+      std::vector<T> w;
+      long nc = 0;  // chunks of 4 taps of the longest line
+    } lm, lt;
+    std::vector<int32_t> lm_base, lm_lidx, lm_row, lt_vox, lt_x0, lt_vl, lt_cls, lt_start{0};
+    long sx = n_int > 0 && sg[0] <= 4 ? sg[0] : 0;
+    if (sx) {
+      struct Run { long lo = LONG_MAX, hi = LONG_MIN; std::vector<int> e; };
+      std::map<std::pair<long, long>, Run> by;  // (dz, dy) -> entries
+      for (int e = 0; e < nD; ++e) {
+        Run& r = by[{d3[3 * e + 2], d3[3 * e + 1]}];
+        r.lo = std::min(r.lo, d3[3 * e]);
+        r.hi = std::max(r.hi, d3[3 * e]);
+        r.e.push_back(e);
+      }
+      for (const auto& kv : by) lm.nc = std::max(lm.nc, (kv.second.hi - kv.second.lo) / 4 + 1);
+      if (lm.nc > kLineChunks) sx = 0;
+      for (const auto& kv : by) {
+        if (!sx) break;
+        const size_t w0 = lm.w.size();
+        lm.w.resize(w0 + 4 * lm.nc, (T)0);
+        for (int e : kv.second.e) lm.w[w0 + (size_t)(d3[3 * e] - kv.second.lo)] = wD[e];
+        lm.off.push_back((int32_t)(kv.second.lo + R0 * kv.first.second + R01 * kv.first.first));
+      }
+    }
+    if (sx) {
+      // items: interior rows in lattice order, each item starts on one
+      std::unordered_map<int32_t, int32_t> at;  // lattice index -> interior row
+      at.reserve(2 * n_int);
+      for (long k = 0; k < n_int; ++k) at[ilidx[k]] = (int32_t)k;
+      std::vector<int32_t> ord(n_int);
+      std::iota(ord.begin(), ord.end(), 0);
+      std::sort(ord.begin(), ord.end(), [&](int32_t a, int32_t b) { return ilidx[a] < ilidx[b]; });
+      int32_t done = INT_MIN;
+      for (int32_t k : ord) {
+        if (ilidx[k] < done) continue;
+        lm_base.push_back(ibase[k]);
+        lm_lidx.push_back(ilidx[k]);
+        for (int i = 0; i < 4; ++i) {
+          // slots past the lattice row's end belong to other lattice points
+          const auto f = at.find(ilidx[k] + i);
+          const bool same = f != at.end() && ibase[f->second] == ibase[k] + sx * i;
+          lm_row.push_back(same ? irow[f->second] : -1);
+        }
+        // the next item starts after this one's slots; a row of another
+        // lattice line among them starts its own
+        done = ilidx[k] + 4;
+        for (int i = 1; i < 4; ++i)
+          if (lm_row[lm_row.size() - 4 + i] < 0 && at.count(ilidx[k] + i)) {
+            done = ilidx[k] + i;
+            break;
+          }
+      }
+      if ((long)lm_base.size() * 2 > n_int) sx = 0;
+      while (lm_base.size() % 64) {
+        lm_base.push_back(lm_base.back());
+        lm_lidx.push_back(lm_lidx.back());
+        lm_row.insert(lm_row.end(), 4, -1);
+      }
+    }
+    if (sx) {
+      const long ub0 = fdiv(-c[0], sx), nug = (fdiv(reg[0] - 1 - c[0], sx) - ub0) / 4 + 1;
+      std::vector<char> hit((size_t)(nug * reg[1] * reg[2]), 0);
+      for (long d = 0; d < n_h; ++d)
+        hit[(fdiv(ijk[3 * d] - c[0], sx) - ub0) / 4 + nug * (ijk[3 * d + 1] + (long)reg[1] * ijk[3 * d + 2])] = 1;
+      struct Run { long lo = LONG_MAX, hi = LONG_MIN; std::vector<int> e; };
+      std::vector<std::map<std::pair<long, long>, Run>> by(sg[1] * sg[2]);  // class -> (oz, oy) -> entries
+      for (int e = 0; e < nD; ++e) {
+        const long cl = fmod_(d3[3 * e + 1], sg[1]) + sg[1] * fmod_(d3[3 * e + 2], sg[2]), o = -fdiv(d3[3 * e], sx);
+        Run& r = by[cl][{-fdiv(d3[3 * e + 2], sg[2]), -fdiv(d3[3 * e + 1], sg[1])}];
+        r.lo = std::min(r.lo, o);
+        r.hi = std::max(r.hi, o);
+        r.e.push_back(e);
+        lt.nc = std::max(lt.nc, (r.hi - r.lo) / 4 + 1);
+      }
+      DR_REQUIRE(lt.nc <= line_chunks((int)sx), DR_ELOGIC, "W stencil: transposed line too long");
+      for (long rz = 0; rz < sg[2]; ++rz)
+        for (long ry = 0; ry < sg[1]; ++ry) {
+          for (const auto& kv : by[ry + sg[1] * rz]) {
+            const size_t w0 = lt.w.size();
+            lt.w.resize(w0 + 4 * sx * lt.nc, (T)0);
+            for (int e : kv.second.e)
+              lt.w[w0 + (size_t)(sx * (-fdiv(d3[3 * e], sx) - kv.second.lo) + fmod_(d3[3 * e], sx))] = wD[e];
+            lt.off.push_back((int32_t)(kv.second.lo + L[0] * (kv.first.second + L[1] * kv.first.first)));
+          }
+          lt_start.push_back((int32_t)lt.off.size());
+          const size_t i0 = lt_vox.size();
+          for (long z = fmod_(c[2] + rz, sg[2]); z < reg[2]; z += sg[2])
+            for (long y = fmod_(c[1] + ry, sg[1]); y < reg[1]; y += sg[1])
+              for (long ug = 0; ug < nug; ++ug) {
+                if (!hit[ug + nug * (y + (long)reg[1] * z)]) continue;
+                const long u[3] = {ub0 + 4 * ug, fdiv(y - c[1], sg[1]), fdiv(z - c[2], sg[2])}, x0 = c[0] + sx * u[0];
+                lt_vox.push_back((int32_t)(x0 + R0 * y + R01 * z));
+                lt_x0.push_back((int32_t)x0);
+                lt_vl.push_back((int32_t)flatL(u));
+              }
+          if (lt_vox.size() > i0)
+            while (lt_vox.size() % 64) {
+              lt_vox.push_back(INT_MIN);
+              lt_x0.push_back(0);
+              lt_vl.push_back(lt_vl.back());
+            }
+          lt_cls.resize(lt_vox.size() / 64, (int32_t)(ry + sg[1] * rz));
+        }
+    }
     // 4. boundary rows: packed offsets from the row's bounding-box corner; v
     //    of boundary row k goes to Vc[k], a compact array.  Rows that span
     //    more than 16 voxels on an axis (the reference's flat-offset
@@ -1211,6 +1330,26 @@ struct Chain : public ChainBase {
           DR_REQUIRE(sub_o[3 * e + a] >= omin[a] && sub_o[3 * e + a] <= omax[a], DR_ELOGIC,
                      "W stencil: sub-stencil offset outside the box margin");
     }
+    if (sx) {  // vector loads of the line kernels, window tails included
+      const long nw = (4 * lm.nc + 3 * sx + 3) / 4 * 4;
+      const auto ends = [](const std::vector<int32_t>& v, size_t a, size_t b) {
+        return std::minmax_element(v.begin() + a, v.begin() + b);
+      };
+      const auto bi = ends(lm_base, 0, lm_base.size()), bo = ends(lm.off, 0, lm.off.size());
+      DR_REQUIRE((long)*bi.first + *bo.first >= 0 && (long)*bi.second + *bo.second + nw - 1 < nreg + kPadR, DR_ELOGIC,
+                 "W stencil: line outside the padded region");
+      for (size_t i = 0; i < lt_vox.size(); i += 64) {
+        const int k = lt_cls[i / 64];
+        if (lt_start[k] == lt_start[k + 1]) continue;
+        const auto vi = ends(lt_vl, i, i + 64), vo = ends(lt.off, lt_start[k], lt_start[k + 1]);
+        DR_REQUIRE((long)*vi.first + *vo.first >= 0 && (long)*vi.second + *vo.second + 4 * lt.nc + 3 < nVl + kPadL,
+                   DR_ELOGIC, "W stencil: line outside the padded lattice grid");
+      }
+      for (size_t i = 0; i < lt_vox.size(); ++i)
+        DR_REQUIRE(lt_vox[i] == INT_MIN ||
+                       (long)lt_vox[i] + 4 * sx - 1 - std::max<long>(0, lt_x0[i] + 4 * sx - reg[0]) < nreg,
+                   DR_ELOGIC, "W stencil: item outside the region");
+    }
     for (size_t k = 0; k < brow.size(); ++k) {
       for (int32_t t = brp[k]; t < brp[k + 1]; ++t) {
         const long q = bd[t], j = (long)bbase[k] + (q & 31) + R0 * ((q >> 5) & 31) + R01 * (q >> 10);
@@ -1260,19 +1399,49 @@ struct Chain : public ChainBase {
       ws.lv[a] = (int)L[a];
     }
     ws.ncls = ncls;
-    upload(ws.irow, mrow);
-    upload(ws.ibase, mbase);
-    upload(ws.ilidx, mlidx);
-    upload(ws.mpar, mpar);
-    upload(ws.wstart, wstart);
-    upload(ws.woff, woff);
-    upload(ws.ww, ww);
+    // W mu by lines from 128 workgroups of 64 items: a wavefront walks a
+    // quarter of the lines one after the other, which only pays once they
+    // fill half of the chip (64x80x64 at 1.5 mm, 42 workgroups in float64:
+    // W mu 23 us by lines, 19 by the window table; 95x113x97, 160 in float32:
+    // 19.3 and 20.1; 1 mm, 380: 88 and 93)
+    const long sxm = (long)lm_base.size() >= 128 * 64 ? sx : 0;
+    ws.sx = (int)sx;
+    ws.sxm = (int)sxm;
+    if (sx) {
+      ws.n_mitem = (int)lm_base.size();
+      ws.n_mline = (int)lm.off.size();
+      ws.n_titem = (int)lt_vox.size();
+      upload(ws.lm_base, lm_base);
+      upload(ws.lm_lidx, lm_lidx);
+      upload(ws.lm_row, lm_row);
+      upload(ws.lm_off, lm.off);
+      ws.nc = (int)lm.nc;
+      upload(ws.lm_w, lm.w);
+      upload(ws.lt_vox, lt_vox);
+      upload(ws.lt_x0, lt_x0);
+      upload(ws.lt_vl, lt_vl);
+      upload(ws.lt_cls, lt_cls);
+      upload(ws.lt_start, lt_start);
+      upload(ws.lt_off, lt.off);
+      ws.mc = (int)lt.nc;
+      upload(ws.lt_w, lt.w);
+    } else {
+      upload(ws.sub_start, sub_start);
+      upload(ws.sub_ldo, sub_ldo);
+      upload(ws.sub_w, sub_w);
+      upload(ws.tiles, tiles);
+    }
+    if (!sxm) {
+      upload(ws.irow, mrow);
+      upload(ws.ibase, mbase);
+      upload(ws.ilidx, mlidx);
+      upload(ws.mpar, mpar);
+      upload(ws.wstart, wstart);
+      upload(ws.woff, woff);
+      upload(ws.ww, ww);
+    }
     ws.n_mslot = (int)mrow.size();
     ws.ncw = (int)ncw;
-    upload(ws.sub_start, sub_start);
-    upload(ws.sub_ldo, sub_ldo);
-    upload(ws.sub_w, sub_w);
-    upload(ws.tiles, tiles);
     upload(ws.brow, brow);
     upload(ws.brp, brp);
     upload(ws.bbase, bbase);
@@ -1292,7 +1461,7 @@ struct Chain : public ChainBase {
     upload(ws.tfw, tfw);
     ws.Vf.alloc(std::max<long>((long)frow.size(), 1));
     ws.Vf.zero(stream);
-    ws.Vl.alloc(std::max<long>(nVl, 1));
+    ws.Vl.alloc(std::max<long>(nVl, 1) + kPadL);
     ws.Vl.zero(stream);
     ws.Vc.alloc(std::max<long>((long)brow.size(), 1));
     ws.Vc.zero(stream);
@@ -1416,26 +1585,60 @@ struct Chain : public ChainBase {
     const int g1 = cdiv(n_s, kThreads / 64);
     const int g2 = cdiv(n_h, kThreads / 16);
     if (use_cls) {
-      const int gi = cdiv((long)ws.n_mslot * kWmuLanes, kThreads), gb = cdiv(ws.n_bnd, kThreads / kWmuBndLanes),
-                gf = cdiv(ws.n_far, kThreads / 64);
+      const int gi = ws.sxm ? ws.n_mitem / 64 : cdiv((long)ws.n_mslot * kWmuLanes, kThreads),
+                gb = cdiv(ws.n_bnd, kThreads / kWmuBndLanes), gf = cdiv(ws.n_far, kThreads / 64);
       if (slot >= 0) note_blocks(slot, gi + gb + gf);
       const int R0 = reg[0], R01 = reg[0] * reg[1];
+      using B = typename Bits<T>::type;
+      // f(lattice step, chunks): the steps 1 to 4 with up to MAXC(step) chunks, or 0, 0
+      auto with_lines = [&](int sx, int nc, auto maxc, auto&& f) {
+        bool found = false;
+        auto step = [&](auto sxc) {
+          constexpr int SX = decltype(sxc)::value, MX = decltype(maxc)::value ? line_chunks(SX) : kLineChunks;
+          auto chunks = [&](auto ncc) {
+            constexpr int NC = decltype(ncc)::value;
+            if constexpr (NC <= MX)
+              if (sx == SX && nc == NC) {
+                f(sxc, ncc);
+                found = true;
+              }
+          };
+          chunks(std::integral_constant<int, 1>{});
+          chunks(std::integral_constant<int, 2>{});
+          chunks(std::integral_constant<int, 3>{});
+          chunks(std::integral_constant<int, 4>{});
+        };
+        if (sx == 0) {
+          f(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
+          return;
+        }
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{});
+        step(std::integral_constant<int, 4>{});
+        DR_REQUIRE(found, DR_ELOGIC, "W products: no kernel for the stencil's lines");
+      };
       if (gi + gb + gf > 0) {
         const WmuInt<T> ai{ws.n_mslot, ws.irow.p, ws.ibase.p, ws.ilidx.p, ws.mpar.p, ws.wstart.p, ws.woff.p,
                            ws.ww.p, ws.ncw, ws.Vl.p};
+        const WmuLines<T> al{ws.n_mitem, ws.n_mline, ws.lm_base.p, ws.lm_lidx.p, ws.lm_row.p, ws.lm_off.p,
+                             reinterpret_cast<const B*>(ws.lm_w.p), ws.Vl.p};
         const WmuBnd<T> ab{ws.n_bnd, ws.brow.p, ws.brp.p, ws.bbase.p, ws.bd.p, ws.bw.p, R0, R01, ws.Vc.p};
         const WmuFar<T> af{ws.n_far, ws.frow.p, ws.frp.p, ws.fcol.p, ws.fw.p, ws.Vf.p};
-        hipLaunchKernelGGL(k_wmu_sb<T>, dim3(gi + gb + gf), dim3(kThreads), (size_t)ws.ncw * (4 + 4 * sizeof(T)), stream,
-                           ai, ab, af, gi, gb, R, Ysd.p, (T)sigma[1], slot >= 0 ? pslot(slot) : nullptr, gsc);
+        const size_t lds = ws.sxm ? 12 * 64 * sizeof(T) : (size_t)ws.ncw * (4 + 4 * sizeof(T));
+        with_lines(ws.sxm, ws.nc, std::false_type{}, [&](auto sxc, auto ncc) {
+          hipLaunchKernelGGL((k_wmu_sb<T, decltype(sxc)::value, decltype(ncc)::value>), dim3(gi + gb + gf), dim3(kThreads), lds, stream, ai,
+                             al, ab, af, gi, gb, R, Ysd.p, (T)sigma[1], slot >= 0 ? pslot(slot) : nullptr, gsc);
+        });
         DR_HIP(hipGetLastError());
       }
       mark();
-      const int ti = ws.n_tiles, tb = cdiv(ws.n_touch, kThreads / kWtvLanes);
+      const int ti = ws.sx ? cdiv(ws.n_titem, kThreads) : ws.n_tiles, tb = cdiv(ws.n_touch, kThreads / kWtvLanes);
       WtvInt<T> wi{};
       wi.tiles = ws.tiles.p;
       wi.cls_start = ws.sub_start.p;
       wi.ldo = ws.sub_ldo.p;
-      wi.w = reinterpret_cast<const typename Bits<T>::type*>(ws.sub_w.p);
+      wi.w = reinterpret_cast<const B*>(ws.sub_w.p);
       wi.Vl = ws.Vl.p;
       wi.mask = mask.p;
       wi.out = WTv.p;
@@ -1450,10 +1653,15 @@ struct Chain : public ChainBase {
         wi.lv[a] = ws.lv[a];
         wi.R[a] = reg[a];
       }
+      const WtvLines<T> wl{ws.n_titem, ws.lt_vox.p, ws.lt_x0.p, ws.lt_vl.p, ws.lt_cls.p, ws.lt_start.p, ws.lt_off.p,
+                           reinterpret_cast<const B*>(ws.lt_w.p), ws.Vl.p, WTv.p, R0};
       const WtvBnd<T> wb{ws.n_touch, ws.tg.p, ws.trp.p, ws.tbase.p, ws.td.p, ws.tw.p, ws.Vc.p, WTvb.p,
                          ws.tfp.p, ws.tfidx.p, ws.tfw.p, ws.Vf.p};
-      const size_t lds_t = (size_t)ws.ldim[0] * ws.ldim[1] * ws.ldim[2] * sizeof(T);
-      hipLaunchKernelGGL(k_wtv_sb<T>, dim3(ti + tb), dim3(kThreads), lds_t, stream, wi, wb, ti);
+      const size_t lds_t = ws.sx ? 0 : (size_t)ws.ldim[0] * ws.ldim[1] * ws.ldim[2] * sizeof(T);
+      with_lines(ws.sx, ws.mc, std::true_type{}, [&](auto sxc, auto mcc) {
+        hipLaunchKernelGGL((k_wtv_sb<T, decltype(sxc)::value, decltype(mcc)::value>), dim3(ti + tb), dim3(kThreads), lds_t, stream, wi, wl,
+                           wb, ti);
+      });
       DR_HIP(hipGetLastError());
       mark();
       return;
@@ -1710,7 +1918,7 @@ struct Chain : public ChainBase {
   void accept_copy(hipStream_t s) {
     DR_HIP(hipMemcpyAsync(muA.p, muB.p, Ns * sizeof(cx<T>), hipMemcpyDeviceToDevice, s));
     if (compat()) DR_HIP(hipMemcpyAsync(miA.p, miB.p, Ns * sizeof(cx<T>), hipMemcpyDeviceToDevice, s));
-    DR_HIP(hipMemcpyAsync(RA.p, RB.p, (nreg + 4) * sizeof(T), hipMemcpyDeviceToDevice, s));
+    DR_HIP(hipMemcpyAsync(RA.p, RB.p, (nreg + kPadR) * sizeof(T), hipMemcpyDeviceToDevice, s));
   }
   // forget captured graphs when buffers move; a batch compares layout_gen
   void drop_graphs() {

@@ -7,6 +7,8 @@
 // the reference (MultiResParameters.h:309-319) with a single array.
 #pragma once
 
+#include <climits>
+
 #include "dr_fft.hpp"
 
 namespace drh {
@@ -632,6 +634,34 @@ template <> struct Bits<double> { using type = uint64_t; };
 __device__ __forceinline__ float from_bits(uint32_t u) { return __uint_as_float(u); }
 __device__ __forceinline__ double from_bits(uint64_t u) { return __longlong_as_double((long long)u); }
 
+// Interior rows by stencil lines: one item is 4 lattice-consecutive rows along
+// x.  A line is the run of stencil entries of one (dy, dz), padded with zero
+// weights to the longest one's chunks of 4 taps.
+template <typename T> struct WmuLines {
+  int nitem, nline;        // items (a multiple of 64); lines
+  const int* base;         // region index of the first row's base
+  const int* lidx;         // its lattice index
+  const int* row;          // 4 rows per item, -1 where the slot holds no interior row
+  const int* loff;         // line: offset of its first tap from a row's base
+  const typename Bits<T>::type* w;  // 4 NC weights per line
+  T* Vl;
+};
+// Interior W^T v by the same lines, transposed: one item is the 4 SX voxels
+// x = c + SX (u + i) + rho, i < 4, rho < SX, of one (y, z); items of one
+// residue class (y mod sg, z mod sg) share their lines.
+template <typename T> struct WtvLines {
+  int nitem;               // items, each class padded to a multiple of 64
+  const int* vox;          // region index of voxel (i, rho) = (0, 0), which may lie left of the row; INT_MIN: padding
+  const int* x0;           // its x
+  const int* vl;           // lattice index of u
+  const int* cls;          // class of each wavefront of items
+  const int* lstart;       // first line of each class
+  const int* loff;         // line: lattice offset of its first tap from u
+  const typename Bits<T>::type* w;  // MC chunks of 4 taps x SX weights per line
+  const T* Vl;
+  T* out;
+  int R0;
+};
 template <typename T> struct WmuInt {
   int n; const int* row; const int* base; const int* lidx; const int* bpar; const int* wstart; const int* woff;
   const T* ww; int ncw; T* Vl;
@@ -733,6 +763,136 @@ __device__ __forceinline__ double wmu_int_block(const WmuInt<T>& a, int blk, con
   return e2;
 }
 
+// 4 consecutive values at any alignment of T
+template <typename T>
+__device__ __forceinline__ void ld4u(const T* p, T* v) {
+  typedef T V __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  const V q = *reinterpret_cast<const V*>(p);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = q[e];
+}
+
+// chunks of 4 taps a line may have: 16 voxels along x, for W^T v in lattice
+// steps of SX (one more where the run does not start on the lattice)
+constexpr int kLineChunks = 4;
+constexpr int line_chunks(int sx) { return sx == 1 ? 4 : sx == 2 ? 3 : 2; }
+
+// Lines l0..l1 (uniform) one after the other: fetch(l, offset) starts a line's
+// vector and weight loads, work() its multiply-adds.  The next line's loads
+// are in flight during a line's arithmetic, the offsets a line further ahead.
+// Every line takes the same number of loads, so that the wait for one line
+// leaves the next one's outstanding (loads under a condition made it wait for
+// all: interior W mu at 1 mm 27 us alone).
+template <class Line, class Fetch, class Work>
+__device__ __forceinline__ void walk_lines(const int* __restrict__ loff, int l0, int l1, Fetch&& fetch, Work&& work) {
+  if (l0 >= l1) return;
+  Line A, B;
+  const int last = l1 - 1;
+  fetch(A, l0, loff[l0]);
+  int on = loff[min(l0 + 1, last)];
+  for (int l = l0; l < l1; l += 2) {
+    const int o2 = loff[min(l + 2, last)];
+    fetch(B, min(l + 1, last), on);
+    work(A);
+    if (l + 1 >= l1) break;
+    on = loff[min(l + 3, last)];
+    fetch(A, min(l + 2, last), o2);
+    work(B);
+  }
+}
+
+// Interior rows by stencil lines: a workgroup takes 64 items, each wavefront a
+// quarter of the lines.  A lane holds a line's voxels in registers and feeds
+// its 4 rows from them: about 5 vector loads for 4 rows of up to 16 taps, with
+// wave-uniform weights from scalar loads, where a row at a time took a load
+// per 4 taps (and the rows were bound by L1 tag lookups).  NC: chunks of 4
+// taps of the longest line.
+template <typename T, int SX, int NC>
+__device__ __forceinline__ double wmu_line_block(const WmuLines<T>& a, int blk, const T* __restrict__ R,
+                                                 const T* __restrict__ Ys, T sig_s) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  T* part = reinterpret_cast<T*>(lds_raw);  // [3][4][64]
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
+  const int it = blk * 64 + ln;
+  const T* Rb = R + a.base[it];
+  constexpr int NW = (4 * NC + 3 * SX + 3) / 4 * 4;  // voxels that 4 NC taps read for 4 rows
+  struct Line { T win[NW], w[4 * NC]; };
+  T acc[4] = {(T)0, (T)0, (T)0, (T)0};
+  walk_lines<Line>(
+      a.loff, a.nline * wv / 4, a.nline * (wv + 1) / 4,
+      [&](Line& x, int l, int off) {
+        const T* q = Rb + off;
+#pragma unroll
+        for (int e = 0; e < NW; e += 4) ld4u(q + e, x.win + e);
+#pragma unroll
+        for (int t = 0; t < 4 * NC; ++t) x.w[t] = from_bits(a.w[4 * NC * l + t]);
+      },
+      [&](const Line& x) {
+#pragma unroll
+        for (int t = 0; t < 4 * NC; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[i] += x.w[t] * x.win[t + SX * i];
+      });
+  if (wv > 0)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) part[((wv - 1) * 4 + i) * 64 + ln] = acc[i];
+  __syncthreads();
+  double e2 = 0.0;
+  if (wv == 0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const T s = (acc[i] + part[i * 64 + ln]) + (part[(4 + i) * 64 + ln] + part[(8 + i) * 64 + ln]);
+      const int row = a.row[4 * it + i];
+      if (row >= 0) {
+        const T e = Ys[row] - s;
+        a.Vl[a.lidx[it] + i] = sig_s * e;
+        e2 += (double)e * (double)e;
+      }
+    }
+  }
+  return e2;
+}
+
+// Interior W^T v by stencil lines: one item (4 SX voxels along x) per lane,
+// its lattice values of a line in registers.  MC: chunks of 4 lattice taps of
+// the longest line.
+template <typename T, int SX, int MC>
+__device__ __forceinline__ void wtv_line_block(const WtvLines<T>& a, int blk) {
+  const int it = blk * kThreads + threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(it >> 6);
+  if (64 * wave >= a.nitem) return;
+  const int g0 = a.vox[it];
+  const T* V = a.Vl + a.vl[it];
+  constexpr int NW = 4 * MC + 4;
+  struct Line { T win[NW], w[4 * SX * MC]; };
+  T acc[4 * SX];
+#pragma unroll
+  for (int i = 0; i < 4 * SX; ++i) acc[i] = (T)0;
+  const int k = a.cls[wave];
+  walk_lines<Line>(
+      a.loff, a.lstart[k], a.lstart[k + 1],
+      [&](Line& x, int l, int off) {
+        const T* q = V + off;
+#pragma unroll
+        for (int e = 0; e < NW; e += 4) ld4u(q + e, x.win + e);
+#pragma unroll
+        for (int t = 0; t < 4 * SX * MC; ++t) x.w[t] = from_bits(a.w[4 * SX * MC * l + t]);
+      },
+      [&](const Line& x) {
+#pragma unroll
+        for (int t = 0; t < 4 * MC; ++t)
+#pragma unroll
+          for (int r = 0; r < SX; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[SX * i + r] += x.w[SX * t + r] * x.win[t + i];
+      });
+  if (g0 == INT_MIN) return;
+  const int x0 = a.x0[it];
+#pragma unroll
+  for (int i = 0; i < 4 * SX; ++i)
+    if (x0 + i >= 0 && x0 + i < a.R0) a.out[g0 + i] = acc[i];
+}
+
 // boundary rows, kWmuBndLanes lanes per row; entry lists start on multiples of 4
 // and are padded to whole quads (offset 0, weight 0)
 template <typename T>
@@ -788,19 +948,24 @@ __device__ __forceinline__ double wmu_far_block(const WmuFar<T>& a, int blk, con
 }
 
 // v = sigma_s (Ys - W R) for every row and ||Ys - W R||^2: blocks [0, gi)
-// take the interior rows, [gi, gi + gb) the packed boundary rows and the rest
-// the far rows, in one launch so the latency-bound gathers and the streaming
-// boundary entries overlap
-template <typename T>
+// take the interior rows (by lines along x where SX, the lattice step, is
+// 1 to 4, else by the window table), [gi, gi + gb) the packed boundary rows
+// and the rest the far rows, in one launch so the interior rows' arithmetic
+// and the streaming boundary entries overlap
+template <typename T, int SX, int NC>
 __global__ void __launch_bounds__(kThreads)
-k_wmu_sb(WmuInt<T> ai, WmuBnd<T> ab, WmuFar<T> af, int gi, int gb, const T* __restrict__ R,
+k_wmu_sb(WmuInt<T> ai, WmuLines<T> al, WmuBnd<T> ab, WmuFar<T> af, int gi, int gb, const T* __restrict__ R,
          const T* __restrict__ Ys, T sig_s, double* part, const StepScalars<T>* sc) {
   __shared__ double red[kThreads];
   if (sc) sig_s = sc->sig1;
   const int blk = blockIdx.x;
-  const double e2 = blk < gi        ? wmu_int_block(ai, blk, R, Ys, sig_s)
-                    : blk < gi + gb ? wmu_bnd_block(ab, blk - gi, R, Ys, sig_s)
-                                    : wmu_far_block(af, blk - gi - gb, R, Ys, sig_s);
+  double e2;
+  if (blk < gi) {
+    if constexpr (SX > 0) e2 = wmu_line_block<T, SX, NC>(al, blk, R, Ys, sig_s);
+    else e2 = wmu_int_block(ai, blk, R, Ys, sig_s);
+  } else {
+    e2 = blk < gi + gb ? wmu_bnd_block(ab, blk - gi, R, Ys, sig_s) : wmu_far_block(af, blk - gi - gb, R, Ys, sig_s);
+  }
   if (part) red_write(e2, red, part, blockIdx.x);
 }
 
@@ -947,11 +1112,16 @@ __device__ __forceinline__ void wtv_bnd_block(const WtvBnd<T>& a, int blk) {
   if (k < a.n && lane == 0) a.out[gj] = acc;
 }
 
-// W^T v: blocks [0, gi) interior voxels, the rest boundary voxels
-template <typename T>
-__global__ void __launch_bounds__(kThreads) k_wtv_sb(WtvInt<T> ai, WtvBnd<T> ab, int gi) {
-  if ((int)blockIdx.x < gi) wtv_int_block(ai, blockIdx.x);
-  else wtv_bnd_block(ab, blockIdx.x - gi);
+// W^T v: blocks [0, gi) interior voxels (by lines for a lattice step SX of 1
+// to 4, else by tiles), the rest boundary voxels
+template <typename T, int SX, int MC>
+__global__ void __launch_bounds__(kThreads) k_wtv_sb(WtvInt<T> ai, WtvLines<T> al, WtvBnd<T> ab, int gi) {
+  if ((int)blockIdx.x < gi) {
+    if constexpr (SX > 0) wtv_line_block<T, SX, MC>(al, blockIdx.x);
+    else wtv_int_block(ai, blockIdx.x);
+  } else {
+    wtv_bnd_block(ab, blockIdx.x - gi);
+  }
 }
 
 // mcmc_summary<T>::update (gaussian_process_model.h:205-224) at the output
