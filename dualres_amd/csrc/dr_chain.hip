@@ -343,7 +343,7 @@ struct Chain : public ChainBase {
     DR_REQUIRE(k_in >= 1 && k_in <= ad.M && k_out >= 1 && k_out <= ad.M && NB >= 1 && n_outer >= 1, DR_ELOGIC,
                "line pass: bad extents");
     if (lines_ok(a, pid)) {
-      const LineArgs<T> la{ad.tw, NB, NB * n_outer, k_in, k_out, src, s_so, dst, d_so, 0};
+      const LineArgs<T> la{ad.tw, NB, NB * n_outer, k_in, k_out, src, s_so, dst, d_so, 0, 0};
       if (INV ? lines_inverse(ad.M, la, stream) : lines_forward(ad.M, la, stream)) {
         mark();
         return;
@@ -536,7 +536,7 @@ struct Chain : public ChainBase {
   void z_inverse(const cx<T>* X) {
     const int NB = M[1] * H0;
     if (lines_ok(2, -1)) {
-      const LineArgs<T> la{axis_dev<T>(2).tw, NB, NB, M[2], reg[2], X, 0, T1.p, 0, M[2]};
+      const LineArgs<T> la{axis_dev<T>(2).tw, NB, NB, M[2], reg[2], X, 0, T1.p, 0, M[2], 0};
       if (lines_inverse(M[2], la, stream)) return;
     }
     strided<T, true>(2, 1, NB, M[2], reg[2], LoadSpec<T>{{}, X, spec()}, StoreS<T>{{}, T1.p, 0, NB});

@@ -1,7 +1,8 @@
 // Instances of the register line transforms (dr_lines.hpp) for every length
 // of DR_LINE_LENGTHS.  Compiled once per precision and pass (DR_LINES_T;
 // DR_LINES_PASS 0 inverse strided, 1 forward strided, 2 leapfrog z, 3 rows
-// without the residual, 4 rows with it) so the objects build side by side.
+// without the residual, 4 rows with it, 5 the correlations, float64 only) so
+// the objects build side by side.
 #include "dr_lines.hpp"
 
 namespace drh {
@@ -20,6 +21,37 @@ int lines_z(int M, const cx<LT>* tw, int nb, int n_in, int n_out, cx<LT>* T1, co
     return g;                                                                                            \
   }
   switch (M) {
+    DR_LINE_LENGTHS(DR_CASE)
+    default: return 0;
+  }
+#undef DR_CASE
+}
+#elif DR_LINES_PASS == 5
+int lines_corr(int M, const CorrZ& a, hipStream_t s) {
+#define DR_CASE(m)                                                                                       \
+  case m: {                                                                                              \
+    using Sh = StridedShape<double, m>;                                                                  \
+    const int g = cdiv(a.nb, Sh::TB);                                                                    \
+    hipLaunchKernelGGL((k_corr_z<m>), dim3(g), dim3(Sh::NT), 0, s, a);                                   \
+    DR_HIP(hipGetLastError());                                                                           \
+    return g;                                                                                            \
+  }
+  switch (M) {
+    DR_LINE_LENGTHS(DR_CASE)
+    default: return 0;
+  }
+#undef DR_CASE
+}
+int rows_mask(int Mh, const MaskRows& a, hipStream_t s) {
+#define DR_CASE(m)                                                                                       \
+  case m: {                                                                                              \
+    using Sh = RowShape<double, m / 2>;                                                                  \
+    const int g = cdiv(a.nrows, Sh::RW);                                                                 \
+    hipLaunchKernelGGL((k_mask_rows<m / 2>), dim3(g), dim3(Sh::NT), 0, s, a);                            \
+    DR_HIP(hipGetLastError());                                                                           \
+    return g;                                                                                            \
+  }
+  switch (2 * Mh) {
     DR_LINE_LENGTHS(DR_CASE)
     default: return 0;
   }

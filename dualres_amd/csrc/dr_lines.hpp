@@ -216,6 +216,7 @@ template <typename T> struct LineArgs {
   cx<T>* dst;
   long d_so;
   int spec;  // rows M2 of a source in the spectral state's layout (one outer index), or 0
+  int wrap;  // also the last `wrap` output rows, stored after the first k_out
 };
 template <typename T, bool INV, int M>
 __global__ void __launch_bounds__((StridedShape<T, M>::NT))
@@ -251,6 +252,7 @@ k_lines(LineArgs<T> a) {
     for (int r = 0; r < RL; ++r) {
       const int k = j + r * BL;
       if (k < a.k_out) d[(unsigned)(k * a.nb)] = v[r];
+      else if (k >= M - a.wrap) d[(unsigned)((k - M + a.wrap + a.k_out) * a.nb)] = v[r];
     }
   }
 }
@@ -562,6 +564,112 @@ __global__ void __launch_bounds__((RowShape<T, Mh>::NT)) k_residual_rows(RowArgs
   }
 }
 
+// ---------------------------------------------------------------- correlations
+// Cross-correlations of an image x and its presence indicator m on a padded
+// torus (dr_mce.hip).  Rows: real samples of x (0 where missing) and m to half
+// spectra.
+struct MaskRows {
+  const cx<double>* tw;  // length-M0 table
+  int nrows, nx;
+  const double* img;     // rows of nx samples; 0 and NaN are missing
+  cx<double>*x, *m;      // half spectra out, row pitch Mh + 1
+};
+template <int Mh>
+__global__ void __launch_bounds__((RowShape<double, Mh>::NT)) k_mask_rows(MaskRows a) {
+  using Sh = RowShape<double, Mh>;
+  using Plan = typename Sh::Plan;
+  constexpr int R1 = Plan::template radix<false>(0), B1 = Mh / R1, RL = Plan::last;
+  __shared__ cx<double> buf[Sh::RW * Sh::P];
+  const int j = threadIdx.x % Plan::nj, l = threadIdx.x / Plan::nj;
+  const int row = blockIdx.x * Sh::RW + l;
+  const bool ok = row < a.nrows;
+  const double* q = a.img + (long)(ok ? row : a.nrows - 1) * a.nx;
+  cx<double> raw[R1], v[Plan::rmax];
+  if (j < B1) {
+#pragma unroll
+    for (int r = 0; r < R1; ++r) {
+      const int x = 2 * (j + r * B1);
+      raw[r] = mk<double>(x < a.nx ? q[x] : 0.0, x + 1 < a.nx ? q[x + 1] : 0.0);
+      if (raw[r].x != raw[r].x) raw[r].x = 0.0;
+      if (raw[r].y != raw[r].y) raw[r].y = 0.0;
+      v[r].x = raw[r].x;
+      v[r].y = raw[r].y;
+    }
+  }
+  auto at = [&](int i) { return &buf[l * Sh::P + Sh::pad(i)]; };
+  line_fft<double, Plan, Mh, false, false, 2>(v, j, a.tw, at, false);
+  row_store_split<double, Mh, RL>(v, j, a.tw, at, ok, a.x + (long)row * (Mh + 1));
+  if (j < B1) {
+#pragma unroll
+    for (int r = 0; r < R1; ++r) {
+      v[r].x = raw[r].x != 0.0 ? 1.0 : 0.0;
+      v[r].y = raw[r].y != 0.0 ? 1.0 : 0.0;
+    }
+  }
+  line_fft<double, Plan, Mh, false, false, 2>(v, j, a.tw, at, true);
+  row_store_split<double, Mh, RL>(v, j, a.tw, at, ok, a.m + (long)row * (Mh + 1));
+}
+
+// z lines: both fields forward, the products conj(X) X, conj(X) M, conj(M) M of
+// every mode, each back to the rows k < k_out and the last `wrap` ones.  One
+// pass over the two fields in place of two forward passes, a product pass and
+// four full inverse ones (x-m and m-x are one field read at p and -p).
+struct CorrZ {
+  const cx<double>* tw;
+  int nb, k_in, k_out, wrap;
+  const cx<double>*x, *m;  // k_in rows of nb columns
+  cx<double>* out[3];      // k_out + wrap rows
+};
+template <int M>
+__global__ void __launch_bounds__((StridedShape<double, M>::NT)) k_corr_z(CorrZ a) {
+  using T = double;
+  using Plan = typename StridedShape<T, M>::Plan;
+  constexpr int TB = StridedShape<T, M>::TB, R1 = Plan::template radix<false>(0), B1 = M / R1, RL = Plan::last;
+  __shared__ cx<T> buf[M * TB];
+  const int b = threadIdx.x % TB, j = threadIdx.x / TB;
+  const int c = xcd_tile(blockIdx.x, gridDim.x) * TB + b;
+  const bool in = c < a.nb;
+  const int cc = in ? c : a.nb - 1;
+  auto at = [&](int i) { return &buf[i * TB + b]; };
+  cx<T> f[2][RL];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const cx<T>* s = (q ? a.m : a.x) + cc;
+    cx<T> v[Plan::rmax];
+    if (j < B1) {
+#pragma unroll
+      for (int r = 0; r < R1; ++r) {
+        v[r] = mk<T>(0, 0);
+        if (r * B1 < a.k_in) {
+          const int k = j + r * B1;
+          const cx<T> x = s[(unsigned)(min(k, a.k_in - 1) * a.nb)];
+          v[r].x = k < a.k_in ? x.x : (T)0;
+          v[r].y = k < a.k_in ? x.y : (T)0;
+        }
+      }
+    }
+    line_fft<T, Plan, M, false, false, 1>(v, j, a.tw, at, q > 0);
+#pragma unroll
+    for (int r = 0; r < RL; ++r) f[q][r] = v[r];
+  }
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    cx<T> v[Plan::rmax];
+#pragma unroll
+    for (int r = 0; r < RL; ++r) v[r] = cmulc(f[p > 0][r], f[p > 1][r]);
+    line_fft<T, Plan, M, true, true, 1>(v, j, a.tw, at, true);
+    if (j < B1 && in) {
+      cx<T>* d = a.out[p] + cc;
+#pragma unroll
+      for (int r = 0; r < R1; ++r) {
+        const int k = j + r * B1;
+        if (k < a.k_out) d[(unsigned)(k * a.nb)] = v[r];
+        else if (k >= M - a.wrap) d[(unsigned)((k - M + a.wrap + a.k_out) * a.nb)] = v[r];
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------- host side
 // Each returns the number of workgroups launched, 0 when no kernel was built
 // for the length (the caller then takes the kernels of dr_fft.hpp).
@@ -576,6 +684,8 @@ __global__ void __launch_bounds__((RowShape<T, Mh>::NT)) k_residual_rows(RowArgs
 DR_LINE_API(float)
 DR_LINE_API(double)
 #undef DR_LINE_API
+int rows_mask(int Mh, const MaskRows& a, hipStream_t s);
+int lines_corr(int M, const CorrZ& a, hipStream_t s);
 
 #define DR_LINE_LENGTHS(X)                                                                                           \
   X(8) X(10) X(12) X(14) X(16) X(18) X(20) X(24) X(28) X(30) X(32) X(36) X(40) X(42) X(48) X(50) X(54) X(56) X(60)    \

@@ -5,10 +5,13 @@
 // that are both present (not 0, not NaN) and inside the image:
 //   Sxy(p) = sum x(u) x(u+p),  Sx(p) = sum x(u),  Sy(p) = sum x(u+p),  n(p).
 // With x the image zeroed where missing and m its presence indicator these
-// are the cross-correlations x*x, x*m, m*x, m*m.  All four come from two
-// forward FFTs (x, m) and four inverse FFTs of conj(A) B on a zero-padded
+// are the cross-correlations x*x, x*m, m*x, m*m on a zero-padded
 // torus larger than the image by the largest offset (no wrap-around), in
-// float64, using the same pass kernels as the sampler.  The per-offset
+// float64.  m*x at p is x*m at -p, so three inverse transforms do; the
+// transforms are pruned to the image on the way in and to the offsets on the
+// way out, and the forward z pass, the products and the inverse z passes are
+// one kernel (corr_lines).  Tori with an axis past the line kernels' lengths
+// take two full forward and four full inverse transforms (corr_full).  The per-offset
 // covariance (Sxy - Sx Sy / n) / (n - 1) is formed on the host, as in the
 // reference, and pair counts are the rounded m*m correlation (exact).
 #include <algorithm>
@@ -18,7 +21,7 @@
 #include <unordered_set>
 #include <vector>
 
-#include "dr_kernels.hpp"
+#include "dr_lines.hpp"
 
 namespace drh {
 
@@ -183,61 +186,141 @@ std::vector<int> mce_offsets() {
   return P;
 }
 
+// read the correlations x*x, x*m, m*m at the offsets p (x*m at -p too) from
+// fields of w2 x w1 rows of M0 samples: an offset's row along an axis is its
+// value modulo w
+__global__ void k_gather_window(int n, const int* __restrict__ off, int M0, int w1, int w2,
+                                const double* __restrict__ R0, const double* __restrict__ R1,
+                                const double* __restrict__ R2, double* __restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  auto at = [&](int s) {
+    const int x = ((s * off[3 * i]) % M0 + M0) % M0, y = ((s * off[3 * i + 1]) % w1 + w1) % w1,
+              z = ((s * off[3 * i + 2]) % w2 + w2) % w2;
+    return x + (long)M0 * (y + (long)w1 * z);
+  };
+  const long g = at(1);
+  out[4 * i] = R0[g];
+  out[4 * i + 1] = R1[g];
+  out[4 * i + 2] = R1[at(-1)];
+  out[4 * i + 3] = R2[g];
+}
+
+struct SumsJob {
+  int dims[3], M[3], reach[3];
+  long n;        // offsets
+  hipStream_t s;
+  const double* img;           // device
+  const int* off;              // device
+  double* out;                 // device, 4 n
+  cx<double>* tw[3];
+};
+
+// the pruned transforms; false when an axis has no line kernel.  One
+// allocation holds every field.
+static bool corr_lines(const SumsJob& j) {
+  const int nx = j.dims[0], ny = j.dims[1], nz = j.dims[2], H0 = j.M[0] / 2 + 1;
+  for (int a = 0; a < 3; ++a)
+    if (j.M[a] > 512 || j.M[a] < 8) return false;
+  // rows kept per axis: offsets 0..reach and -reach..-1, or all of them
+  int ko[3], wr[3], w[3];
+  for (int a = 1; a < 3; ++a) {
+    const bool all = 2 * j.reach[a] + 1 >= j.M[a];
+    ko[a] = all ? j.M[a] : j.reach[a] + 1;
+    wr[a] = all ? 0 : j.reach[a];
+    w[a] = ko[a] + wr[a];
+  }
+  const long rows = (long)ny * nz, tx = rows * H0, ty = (long)nz * j.M[1] * H0, tz = (long)w[2] * j.M[1] * H0,
+             tw = (long)w[2] * w[1] * H0, tr = (long)w[2] * w[1] * j.M[0];
+  if (std::max(ty, tz) * (long)sizeof(cx<double>) >= (1L << 31)) return false;
+  // A: half spectra of the rows (x, m), then of the kept rows; B: after the y
+  // pass (x, m); C: after the z pass (3 fields); R: samples
+  const long nA = std::max(2 * tx, 3 * tw), nB = 2 * ty, nC = 3 * tz;
+  MBuf<cx<double>> ws(nA + nB + nC + (3 * tr + 1) / 2);
+  cx<double>*A = ws.p, *B = A + nA, *C = B + nB;
+  double* R = reinterpret_cast<double*>(C + nC);
+  auto need = [](int g) { DR_REQUIRE(g > 0, DR_ELOGIC, "minimum contrast: no line kernel for this length"); };
+  need(rows_mask(j.M[0] / 2, MaskRows{j.tw[0], (int)rows, nx, j.img, A, A + tx}, j.s));
+  for (int q = 0; q < 2; ++q)
+    need(lines_forward(j.M[1], LineArgs<double>{j.tw[1], H0, H0 * nz, ny, j.M[1], A + q * tx, (long)ny * H0,
+                                                B + q * ty, (long)j.M[1] * H0, 0, 0}, j.s));
+  need(lines_corr(j.M[2], CorrZ{j.tw[2], j.M[1] * H0, nz, ko[2], wr[2], B, B + ty, {C, C + tz, C + 2 * tz}}, j.s));
+  // the three fields are one batch of 3 w2 planes
+  need(lines_inverse(j.M[1], LineArgs<double>{j.tw[1], H0, H0 * 3 * w[2], j.M[1], ko[1], C, (long)j.M[1] * H0, A,
+                                              (long)w[1] * H0, 0, wr[1]}, j.s));
+  const double scale = 1.0 / ((double)j.M[0] * j.M[1] * j.M[2]);
+  need(rows_c2r(j.M[0] / 2, RowArgs<double>{j.tw[0], 3 * w[2] * w[1], j.M[0], A, nullptr, R, scale}, j.s));
+  hipLaunchKernelGGL(k_gather_window, dim3(cdiv(j.n, 256)), dim3(256), 0, j.s, (int)j.n, j.off, j.M[0], w[1], w[2], R,
+                     R + tr, R + 2 * tr, j.out);
+  DR_HIP(hipGetLastError());
+  DR_HIP(hipStreamSynchronize(j.s));  // the workspace is freed on return
+  return true;
+}
+
+static void corr_full(const SumsJob& j) {
+  const int* M = j.M;
+  long N, Nh;
+  Fft3d::sizes(M, &N, &Nh);
+  MBuf<cx<double>> T1(Nh), T2(Nh), X(Nh), Mk(Nh), P[4];
+  Fft3d f;
+  f.plan(M, j.s, j.tw, T1.p, T2.p);
+  f.r2c(LoadMasked{{}, j.img, j.dims[0], j.dims[1], j.dims[2], M[1], 0}, X.p);
+  f.r2c(LoadMasked{{}, j.img, j.dims[0], j.dims[1], j.dims[2], M[1], 1}, Mk.p);
+  for (auto& q : P) q.alloc(Nh);
+  hipLaunchKernelGGL(k_corr_products, dim3(cdiv(Nh, 256)), dim3(256), 0, j.s, Nh, X.p, Mk.p, P[0].p, P[1].p, P[2].p,
+                     P[3].p);
+  DR_HIP(hipGetLastError());
+  MBuf<double> R[4];
+  for (int k = 0; k < 4; ++k) {
+    R[k].alloc(N);
+    f.c2r(P[k].p, R[k].p);
+  }
+  hipLaunchKernelGGL(k_gather_offsets, dim3(cdiv(j.n, 256)), dim3(256), 0, j.s, (int)j.n, j.off, M[0], M[1], M[2],
+                     R[0].p, R[1].p, R[2].p, R[3].p, j.out);
+  DR_HIP(hipGetLastError());
+  DR_HIP(hipStreamSynchronize(j.s));
+}
+
 // correlation sums (Sxy, Sx, Sy, n) at each offset, float64
 static std::vector<double> corr_sums(const double* img, const int dims[3], const std::vector<int>& off, int device) {
   DR_REQUIRE(img && dims, DR_ELOGIC, "minimum contrast: null argument");
   for (int a = 0; a < 3; ++a) DR_REQUIRE(dims[a] >= 1, DR_EDOMAIN, "minimum contrast: empty image");
-  int reach[3] = {0, 0, 0};
-  const long n = (long)off.size() / 3;
-  for (long i = 0; i < n; ++i)
-    for (int a = 0; a < 3; ++a) reach[a] = std::max(reach[a], std::abs(off[3 * i + a]));
-  int M[3];
+  SumsJob j{};
+  j.n = (long)off.size() / 3;
+  for (long i = 0; i < j.n; ++i)
+    for (int a = 0; a < 3; ++a) j.reach[a] = std::max(j.reach[a], std::abs(off[3 * i + a]));
   for (int a = 0; a < 3; ++a) {
-    M[a] = smooth_even(dims[a] + reach[a] + 1);
-    DR_REQUIRE(M[a] <= 2048, DR_EDOMAIN, "minimum contrast: image axis too long");
+    j.dims[a] = dims[a];
+    j.M[a] = smooth_even(dims[a] + j.reach[a] + 1);
+    DR_REQUIRE(j.M[a] <= 2048, DR_EDOMAIN, "minimum contrast: image axis too long");
   }
   DR_HIP(hipSetDevice(device));
-  hipStream_t s;
-  DR_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-  struct SG { hipStream_t s; ~SG() { (void)hipStreamSynchronize(s); (void)hipStreamDestroy(s); } } sg{s};
-  long N, Nh;
-  Fft3d::sizes(M, &N, &Nh);
-  MBuf<cx<double>> tw[3], T1(Nh), T2(Nh);
-  cx<double>* twp[3];
+  DR_HIP(hipStreamCreateWithFlags(&j.s, hipStreamNonBlocking));
+  struct SG { hipStream_t s; ~SG() { (void)hipStreamSynchronize(s); (void)hipStreamDestroy(s); } } sg{j.s};
+  // one allocation: image, twiddles, offsets, sums
+  const long nvox = (long)dims[0] * dims[1] * dims[2], ntw = 2L * (j.M[0] + j.M[1] + j.M[2]);
+  MBuf<double> in(nvox + 1 + ntw + 4 * j.n + (3 * j.n + 1) / 2 + 4);
+  double* at = in.p + (nvox + 1) / 2 * 2;  // complex values stay aligned
+  std::vector<double> tw;
   for (int a = 0; a < 3; ++a) {
-    const auto t = twiddles<double>(M[a]);
-    tw[a].alloc(M[a]);
-    DR_HIP(hipMemcpyAsync(tw[a].p, t.data(), M[a] * sizeof(cx<double>), hipMemcpyHostToDevice, s));
-    DR_HIP(hipStreamSynchronize(s));
-    twp[a] = tw[a].p;
+    j.tw[a] = reinterpret_cast<cx<double>*>(at + tw.size());
+    for (const cx<double>& t : twiddles<double>(j.M[a])) {
+      tw.push_back(t.x);
+      tw.push_back(t.y);
+    }
   }
-  Fft3d f;
-  f.plan(M, s, twp, T1.p, T2.p);
-  const long nvox = (long)dims[0] * dims[1] * dims[2];
-  MBuf<double> d_img(nvox);
-  DR_HIP(hipMemcpyAsync(d_img.p, img, nvox * sizeof(double), hipMemcpyHostToDevice, s));
-  MBuf<cx<double>> X(f.Nh), Mk(f.Nh), P[4];
-  f.r2c(LoadMasked{{}, d_img.p, dims[0], dims[1], dims[2], M[1], 0}, X.p);
-  f.r2c(LoadMasked{{}, d_img.p, dims[0], dims[1], dims[2], M[1], 1}, Mk.p);
-  for (auto& q : P) q.alloc(f.Nh);
-  hipLaunchKernelGGL(k_corr_products, dim3(cdiv(f.Nh, 256)), dim3(256), 0, s, f.Nh, X.p, Mk.p, P[0].p, P[1].p,
-                     P[2].p, P[3].p);
-  DR_HIP(hipGetLastError());
-  MBuf<double> R[4];
-  for (int k = 0; k < 4; ++k) {
-    R[k].alloc(f.N);
-    f.c2r(P[k].p, R[k].p);
-  }
-  MBuf<int> d_off(off.size());
-  MBuf<double> d_out(4 * n);
-  DR_HIP(hipMemcpyAsync(d_off.p, off.data(), off.size() * sizeof(int), hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_gather_offsets, dim3(cdiv(n, 256)), dim3(256), 0, s, (int)n, d_off.p, M[0], M[1], M[2], R[0].p,
-                     R[1].p, R[2].p, R[3].p, d_out.p);
-  DR_HIP(hipGetLastError());
-  std::vector<double> out(4 * n);
-  DR_HIP(hipMemcpyAsync(out.data(), d_out.p, 4 * n * sizeof(double), hipMemcpyDeviceToHost, s));
-  DR_HIP(hipStreamSynchronize(s));
-  for (long i = 0; i < n; ++i) out[4 * i + 3] = std::nearbyint(out[4 * i + 3]);
+  j.img = in.p;
+  j.out = at + ntw;
+  int* d_off = reinterpret_cast<int*>(j.out + 4 * j.n);
+  j.off = d_off;
+  DR_HIP(hipMemcpyAsync(at, tw.data(), tw.size() * sizeof(double), hipMemcpyHostToDevice, j.s));
+  DR_HIP(hipMemcpyAsync(d_off, off.data(), off.size() * sizeof(int), hipMemcpyHostToDevice, j.s));
+  DR_HIP(hipMemcpyAsync(in.p, img, nvox * sizeof(double), hipMemcpyHostToDevice, j.s));
+  if (!corr_lines(j)) corr_full(j);
+  std::vector<double> out(4 * j.n);
+  DR_HIP(hipMemcpyAsync(out.data(), j.out, 4 * j.n * sizeof(double), hipMemcpyDeviceToHost, j.s));
+  DR_HIP(hipStreamSynchronize(j.s));
+  for (long i = 0; i < j.n; ++i) out[4 * i + 3] = std::nearbyint(out[4 * i + 3]);
   return out;
 }
 
