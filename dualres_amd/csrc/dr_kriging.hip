@@ -1196,14 +1196,22 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
   std::vector<uint8_t> present(nvox);
   int lo[3] = {nx, ny, nz}, hi[3] = {-1, -1, -1};
   long nnz_hr = 0;
-  for (long f = 0; f < nvox; ++f) {
-    present[f] = pres(hr[f]);
-    if (present[f]) {
-      const int c[3] = {(int)(f % nx), (int)((f / nx) % ny), (int)(f / ((long)nx * ny))};
-      for (int a = 0; a < 3; ++a) { lo[a] = std::min(lo[a], c[a]); hi[a] = std::max(hi[a], c[a]); }
-      ++nnz_hr;
+  for (int k = 0; k < nz; ++k)
+    for (int j = 0; j < ny; ++j) {
+      const long f0 = (long)nx * (j + (long)ny * k);
+      int first = nx, last = -1;
+      for (int i = 0; i < nx; ++i) {
+        const bool p = pres(hr[f0 + i]);
+        present[f0 + i] = p;
+        if (!p) continue;
+        first = std::min(first, i);
+        last = i;
+        ++nnz_hr;
+      }
+      if (last < 0) continue;
+      const int a[3] = {first, j, k}, b[3] = {last, j, k};
+      for (int c = 0; c < 3; ++c) { lo[c] = std::min(lo[c], a[c]); hi[c] = std::max(hi[c], b[c]); }
     }
-  }
   DR_REQUIRE(nnz_hr > 0, DR_EDOMAIN, "kriging_build: high-resolution image has no nonzero voxels");
   int bd[3];
   for (int a = 0; a < 3; ++a) bd[a] = hi[a] - lo[a] + 1;
@@ -1219,14 +1227,12 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
         }
   }
   // stdres nonzero ijk (nifti_manipulation.inl:334-360)
-  const long snvox = (long)sdims[0] * sdims[1] * sdims[2];
   std::vector<int> sijk;
-  for (long f = 0; f < snvox; ++f)
-    if (pres(st[f])) {
-      sijk.push_back((int)(f % sdims[0]));
-      sijk.push_back((int)((f / sdims[0]) % sdims[1]));
-      sijk.push_back((int)(f / ((long)sdims[0] * sdims[1])));
-    }
+  long sf = 0;
+  for (int k = 0; k < sdims[2]; ++k)
+    for (int j = 0; j < sdims[1]; ++j)
+      for (int i = 0; i < sdims[0]; ++i)
+        if (pres(st[sf++])) sijk.insert(sijk.end(), {i, j, k});
   const int n_rows = (int)(sijk.size() / 3);
   DR_REQUIRE(n_rows > 0, DR_EDOMAIN, "kriging_build: standard-resolution image has no nonzero voxels");
   // map = Qh^-1 Qs (float32 rounding of the float64 product)
@@ -1295,6 +1301,7 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
   struct Key { uint64_t a, b; int n; bool operator==(const Key& o) const { return a == o.a && b == o.b && n == o.n; } };
   struct KH { size_t operator()(const Key& k) const { return (size_t)(k.a ^ (k.b * 31) ^ (uint64_t)k.n); } };
   std::unordered_map<Key, int, KH> seen;
+  seen.reserve(n_rows);
   std::vector<int> rep(n_rows), uid(n_rows), urow;
   for (int i = 0; i < n_rows; ++i) {
     if (cnt[i] == 0) { rep[i] = i; uid[i] = -1; continue; }

@@ -162,7 +162,7 @@ struct Fft3d {
 }  // namespace
 
 // unique MCE offsets in first-occurrence order (perturbation_matrix.h:20-106)
-std::vector<int> mce_offsets() {
+static std::vector<int> make_mce_offsets() {
   static const int U[14][3] = {{0, 0, 0},  {1, 0, 0},  {0, 1, 0},  {0, 0, 1},  {1, 1, 0},
                                {1, 0, 1},  {-1, 1, 0}, {1, 0, -1}, {0, 1, 1},  {0, 1, -1},
                                {1, 1, 1},  {1, 1, -1}, {-1, 1, 1}, {-1, 1, -1}};
@@ -183,6 +183,12 @@ std::vector<int> mce_offsets() {
       v[j] = na + i + 1;
       push(v[0], v[1], v[2]);
     }
+  return P;
+}
+
+// The table is the same for every image: built once per process (1 ms).
+const std::vector<int>& mce_offsets() {
+  static const std::vector<int> P = make_mce_offsets();
   return P;
 }
 
@@ -370,7 +376,7 @@ static const NoAllocDevice& noalloc_setup(int device) {
   p = nullptr;
   DR_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(mce_offset_table)));
   d.off = static_cast<int*>(p);
-  const std::vector<int> P = mce_offsets();
+  const std::vector<int>& P = mce_offsets();
   DR_REQUIRE((long)P.size() == 3L * kNumMceOffsets, DR_ELOGIC, "minimum contrast: offset table size changed");
   DR_HIP(hipMemcpy(d.off, P.data(), P.size() * sizeof(int), hipMemcpyHostToDevice));
   d.ready = true;
@@ -461,7 +467,7 @@ extern "C" {
 int dr_mce_offsets(int64_t* n, int32_t* offsets_xyz) {
   return drh::guarded([&] {
     DR_REQUIRE(n, DR_ELOGIC, "dr_mce_offsets: null count");
-    const std::vector<int> P = drh::mce_offsets();
+    const std::vector<int>& P = drh::mce_offsets();
     *n = (int64_t)(P.size() / 3);
     if (offsets_xyz) std::copy(P.begin(), P.end(), offsets_xyz);
   });
@@ -471,7 +477,7 @@ int dr_mce_summary(const double* img, const int dims[3], const float qform[16], 
                    float* distance, int32_t* npairs) {
   return drh::guarded([&] {
     DR_REQUIRE(covariance && distance && npairs && qform, DR_ELOGIC, "dr_mce_summary: null output");
-    const std::vector<int> P = drh::mce_offsets();
+    const std::vector<int>& P = drh::mce_offsets();
     const std::vector<double> s = drh::corr_sums(img, dims, P, device);
     const long n = (long)P.size() / 3;
     for (long i = 0; i < n; ++i) {

@@ -6,13 +6,17 @@ import numpy as np
 from . import _lib as L
 
 
+def _n_offsets(lib):
+    n = C.c_int64()
+    L.check(lib.dr_mce_offsets(C.byref(n), None))
+    return n.value
+
+
 def mce_offsets():
     """The reference's 25,348 voxel offsets (perturbation_matrix.h:62-106), (n, 3) int."""
     lib = L.load()
-    n = C.c_int64()
-    L.check(lib.dr_mce_offsets(C.byref(n), None))
-    out = np.empty((n.value, 3), dtype=np.int32)
-    L.check(lib.dr_mce_offsets(C.byref(n), L.iptr32(out)))
+    out = np.empty((_n_offsets(lib), 3), dtype=np.int32)
+    L.check(lib.dr_mce_offsets(C.byref(C.c_int64()), L.iptr32(out)))
     return out
 
 
@@ -24,7 +28,7 @@ def mce_summary(img, qform, device=0):
     """(covariance f32, distance f32, npairs i32) per offset; img shape (nz, ny, nx)."""
     lib = L.load()
     img = np.ascontiguousarray(img, dtype=np.float64)
-    n = mce_offsets().shape[0]
+    n = _n_offsets(lib)
     cov = np.empty(n, np.float32)
     dist = np.empty(n, np.float32)
     npairs = np.empty(n, np.int32)
