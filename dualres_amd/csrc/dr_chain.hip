@@ -1716,6 +1716,7 @@ struct Chain : public ChainBase {
   // transformed back into T1.  A single-resolution residual is local to a row
   // and takes one kernel on T2 in place, which writes mu to R only if keep.
   void likelihood(T* R, int slot_h, int slot_s, bool keep) {
+    if (cfg.n_datasets == 1 && planes(row_args(keep ? R : nullptr), residual(R, slot_h), slot_h)) return;
     if (cfg.n_datasets == 1 && lines_ok(0, P_XI) && lines_ok(0, P_XF)) {
       y_inverse();
       if (const int g = rows_residual(M[0] / 2, row_args(keep ? R : nullptr), residual(R, slot_h), stream)) {
@@ -1732,6 +1733,18 @@ struct Chain : public ChainBase {
     }
     w_products(R, slot_s);
     r2c_xy(residual(R, slot_h), slot_h);
+  }
+  // the same by planes, for the tori that have a kernel; false: nothing ran
+  bool planes(const RowArgs<T>& x, const LoadResidual<T>& res, int slot) {
+    for (int pid : {P_YI, P_YF})
+      if (!lines_ok(1, pid)) return false;
+    for (int pid : {P_XI, P_XF})
+      if (!lines_ok(0, pid)) return false;
+    const PlaneArgs<T> a{axis_dev<T>(1).tw, reg[1], T1.p, x};
+    if (!plane_residual(M[0] / 2, M[1], reg[2], a, res, stream)) return false;
+    if (slot >= 0) note_blocks(slot, reg[2]);
+    for (int i = 0; i < 4; ++i) mark();  // the y, x, x and y passes of the profile
+    return true;
   }
   RowArgs<T> row_args(T* R) {
     return RowArgs<T>{axis_dev<T>(0).tw, reg[1] * reg[2], reg[0], T2.p, T2.p, R, (T)(1.0 / (double)N)};

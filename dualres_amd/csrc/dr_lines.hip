@@ -1,8 +1,8 @@
 // Instances of the register line transforms (dr_lines.hpp) for every length
 // of DR_LINE_LENGTHS.  Compiled once per precision and pass (DR_LINES_T;
 // DR_LINES_PASS 0 inverse strided, 1 forward strided, 2 leapfrog z, 3 rows
-// without the residual, 4 rows with it, 5 the correlations, float64 only) so
-// the objects build side by side.
+// without the residual, 4 rows with it, 5 the correlations, float64 only, 6
+// whole planes) so the objects build side by side.
 #include "dr_lines.hpp"
 
 namespace drh {
@@ -56,6 +56,29 @@ int rows_mask(int Mh, const MaskRows& a, hipStream_t s) {
     default: return 0;
   }
 #undef DR_CASE
+}
+#elif DR_LINES_PASS == 6
+template <int m0, int m1>
+static bool plane_launch(int nz, const PlaneArgs<LT>& a, const RowResidual<LT>& rr, hipStream_t s) {
+  if constexpr (m0 * m1 <= plane_cap<LT>()) {
+    hipLaunchKernelGGL((k_plane<LT, m0 / 2, m1>), dim3(nz), dim3(kPlaneNT), 0, s, a, rr);
+    DR_HIP(hipGetLastError());
+    return true;
+  }
+  return false;
+}
+// the region's rows have to fit in the kernel's plane (they do where the
+// torus is at least twice the data) and samples are fetched in pairs
+int plane_residual(int Mh, int MY, int nz, const PlaneArgs<LT>& a, const LoadResidual<LT>& res, hipStream_t s) {
+  if (a.x.n0 < 2 || a.n1 < 1 || a.n1 > MY / 2 + 1) return 0;
+  const RowResidual<LT> rr{res};
+#define DR_CASE(m0, m1) \
+  if (2 * Mh == m0 && MY == m1) return plane_launch<m0, m1>(nz, a, rr, s) ? nz : 0;
+#define DR_ROW(m0) DR_CASE(m0, 32) DR_CASE(m0, 48) DR_CASE(m0, 64) DR_CASE(m0, 96) DR_CASE(m0, 128)
+  DR_ROW(32) DR_ROW(48) DR_ROW(64) DR_ROW(96) DR_ROW(128)
+#undef DR_ROW
+#undef DR_CASE
+  return 0;
 }
 #elif DR_LINES_PASS < 2
 #if DR_LINES_PASS == 0

@@ -443,24 +443,23 @@ template <typename T> struct RowArgs {
   T scale;          // 1 / N
 };
 
-// half spectra -> scaled samples
-template <typename T, int Mh>
-__global__ void __launch_bounds__((RowShape<T, Mh>::NT)) k_c2r_rows(RowArgs<T> a) {
-  using Sh = RowShape<T, Mh>;
-  using Plan = typename Sh::Plan;
+// One row of a group whose lanes run along it: j counts the row's threads
+// (plan nj of them), at(i) is the LDS slot of element i, X the half spectrum
+// read and D the one written (which may be X), row the row's number in the
+// region; ok is false for a lane past the last row, which works on a row it
+// must not store to.
+// half spectrum -> scaled samples
+template <typename T, int Mh, class At>
+__device__ __forceinline__ void row_inverse(const RowArgs<T>& a, const cx<T>* X, int row, int j, bool ok, At&& at,
+                                            bool war) {
+  using Plan = typename RowShape<T, Mh>::Plan;
   constexpr int R1 = Plan::template radix<false>(0), B1 = Mh / R1, RL = Plan::last, BL = Mh / RL;
-  __shared__ cx<T> buf[Sh::RW * Sh::P];
-  const int j = threadIdx.x % Plan::nj, l = threadIdx.x / Plan::nj;
-  const int row = blockIdx.x * Sh::RW + l;
-  const bool ok = row < a.nrows;
-  const int rc = ok ? row : a.nrows - 1;
   cx<T> v[Plan::rmax];
   if (j < B1) {
-    const cx<T>* X = a.src + (long)rc * (Mh + 1);
 #pragma unroll
     for (int r = 0; r < R1; ++r) v[r] = row_merge<T, Mh>(X, a.tw, j + r * B1);
   }
-  line_fft<T, Plan, Mh, true, false, 2>(v, j, a.tw, [&](int i) { return &buf[l * Sh::P + Sh::pad(i)]; }, false);
+  line_fft<T, Plan, Mh, true, false, 2>(v, j, a.tw, at, war);
   if (j < BL && ok) {
     T* d = a.R + (long)row * a.n0;
 #pragma unroll
@@ -472,18 +471,12 @@ __global__ void __launch_bounds__((RowShape<T, Mh>::NT)) k_c2r_rows(RowArgs<T> a
   }
 }
 
-// residual rows -> half spectra
-template <typename T, int Mh>
-__global__ void __launch_bounds__((RowShape<T, Mh>::NT)) k_r2c_rows(RowArgs<T> a, RowResidual<T> res) {
-  using Sh = RowShape<T, Mh>;
-  using Plan = typename Sh::Plan;
+// residual of the row's samples -> half spectrum
+template <typename T, int Mh, class At>
+__device__ __forceinline__ void row_forward(const RowArgs<T>& a, RowResidual<T>& res, cx<T>* D, int row, int j,
+                                            bool ok, At&& at, bool war) {
+  using Plan = typename RowShape<T, Mh>::Plan;
   constexpr int R1 = Plan::template radix<false>(0), B1 = Mh / R1, RL = Plan::last;
-  __shared__ __align__(16) cx<T> buf[Sh::RW * Sh::P < Sh::NT ? Sh::NT : Sh::RW * Sh::P];
-  bind_scalars(res.q);
-  const int j = threadIdx.x % Plan::nj, l = threadIdx.x / Plan::nj;
-  const int row = blockIdx.x * Sh::RW + l;
-  const bool ok = row < a.nrows;
-  const int rc = ok ? row : a.nrows - 1;
   cx<T> v[Plan::rmax];
   if (j < B1) {
 #pragma unroll
@@ -491,7 +484,7 @@ __global__ void __launch_bounds__((RowShape<T, Mh>::NT)) k_r2c_rows(RowArgs<T> a
       typename RowResidual<T>::In in[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u)
-        if (r0 + u < R1 && 2 * (r0 + u) * B1 < a.n0) in[u] = res.template fetch<true>(rc, j + (r0 + u) * B1);
+        if (r0 + u < R1 && 2 * (r0 + u) * B1 < a.n0) in[u] = res.template fetch<true>(row, j + (r0 + u) * B1);
 #pragma unroll
       for (int u = 0; u < 4; ++u)
         if (r0 + u < R1) {
@@ -500,45 +493,32 @@ __global__ void __launch_bounds__((RowShape<T, Mh>::NT)) k_r2c_rows(RowArgs<T> a
         }
     }
   }
-  auto at = [&](int i) { return &buf[l * Sh::P + Sh::pad(i)]; };
-  line_fft<T, Plan, Mh, false, false, 2>(v, j, a.tw, at, false);
-  row_store_split<T, Mh, RL>(v, j, a.tw, at, ok, a.dst + (long)rc * (Mh + 1));
-  if (res.q.part) {
-    const double s = line_sum<Sh::NT>(res.q.acc, reinterpret_cast<double*>(buf));
-    if (threadIdx.x == 0) res.q.part[blockIdx.x] = s;
-  }
+  line_fft<T, Plan, Mh, false, false, 2>(v, j, a.tw, at, war);
+  row_store_split<T, Mh, RL>(v, j, a.tw, at, ok, D);
 }
 
-// half spectra -> samples -> residual -> half spectra, in place: without W
-// the likelihood is local to a row.  mu goes to R only where it is asked for.
+// half spectrum -> samples -> residual -> half spectrum: without W the
+// likelihood is local to a row.  mu goes to R only where it is asked for.
 // The way back runs the stages in the opposite order, so it starts on the
 // samples the inverse transform left in the thread's registers.
-template <typename T, int Mh>
-__global__ void __launch_bounds__((RowShape<T, Mh>::NT)) k_residual_rows(RowArgs<T> a, RowResidual<T> res) {
-  using Sh = RowShape<T, Mh>;
-  using Plan = typename Sh::Plan;
+template <typename T, int Mh, class At>
+__device__ __forceinline__ void row_residual(const RowArgs<T>& a, RowResidual<T>& res, const cx<T>* X, cx<T>* D,
+                                             int row, int j, bool ok, At&& at, bool war) {
+  using Plan = typename RowShape<T, Mh>::Plan;
   constexpr int R1 = Plan::template radix<false>(0), B1 = Mh / R1, RL = Plan::last, BL = Mh / RL;
-  __shared__ __align__(16) cx<T> buf[Sh::RW * Sh::P < Sh::NT ? Sh::NT : Sh::RW * Sh::P];
-  bind_scalars(res.q);
-  const int j = threadIdx.x % Plan::nj, l = threadIdx.x / Plan::nj;
-  const int row = blockIdx.x * Sh::RW + l;
-  const bool ok = row < a.nrows;
-  const int rc = ok ? row : a.nrows - 1;
   cx<T> v[Plan::rmax];
   if (j < B1) {
-    const cx<T>* X = a.src + (long)rc * (Mh + 1);
 #pragma unroll
     for (int r = 0; r < R1; ++r) v[r] = row_merge<T, Mh>(X, a.tw, j + r * B1);
   }
-  auto at = [&](int i) { return &buf[l * Sh::P + Sh::pad(i)]; };
-  line_fft<T, Plan, Mh, true, false, 2>(v, j, a.tw, at, false);
+  line_fft<T, Plan, Mh, true, false, 2>(v, j, a.tw, at, war);
   // BL is the widest stage: every thread owns RL packed samples
 #pragma unroll
   for (int r0 = 0; r0 < RL; r0 += 4) {
     typename RowResidual<T>::In in[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      if (r0 + u < RL && 2 * (r0 + u) * BL < a.n0) in[u] = res.template fetch<false>(rc, j + (r0 + u) * BL);
+      if (r0 + u < RL && 2 * (r0 + u) * BL < a.n0) in[u] = res.template fetch<false>(row, j + (r0 + u) * BL);
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       if (r0 + u < RL) {
@@ -557,10 +537,140 @@ __global__ void __launch_bounds__((RowShape<T, Mh>::NT)) k_residual_rows(RowArgs
       }
   }
   line_fft<T, Plan, Mh, false, true, 2>(v, j, a.tw, at, true);
-  row_store_split<T, Mh, R1>(v, j, a.tw, at, ok, a.dst + (long)rc * (Mh + 1));
+  row_store_split<T, Mh, R1>(v, j, a.tw, at, ok, D);
+}
+
+template <typename T, int Mh>
+__global__ void __launch_bounds__((RowShape<T, Mh>::NT)) k_c2r_rows(RowArgs<T> a) {
+  using Sh = RowShape<T, Mh>;
+  __shared__ cx<T> buf[Sh::RW * Sh::P];
+  const int j = threadIdx.x % Sh::Plan::nj, l = threadIdx.x / Sh::Plan::nj;
+  const int row = blockIdx.x * Sh::RW + l, rc = min(row, a.nrows - 1);
+  row_inverse<T, Mh>(a, a.src + (long)rc * (Mh + 1), rc, j, row < a.nrows,
+                     [&](int i) { return &buf[l * Sh::P + Sh::pad(i)]; }, false);
+}
+
+template <typename T, int Mh>
+__global__ void __launch_bounds__((RowShape<T, Mh>::NT)) k_r2c_rows(RowArgs<T> a, RowResidual<T> res) {
+  using Sh = RowShape<T, Mh>;
+  __shared__ __align__(16) cx<T> buf[Sh::RW * Sh::P < Sh::NT ? Sh::NT : Sh::RW * Sh::P];
+  bind_scalars(res.q);
+  const int j = threadIdx.x % Sh::Plan::nj, l = threadIdx.x / Sh::Plan::nj;
+  const int row = blockIdx.x * Sh::RW + l, rc = min(row, a.nrows - 1);
+  row_forward<T, Mh>(a, res, a.dst + (long)rc * (Mh + 1), rc, j, row < a.nrows,
+                     [&](int i) { return &buf[l * Sh::P + Sh::pad(i)]; }, false);
   if (res.q.part) {
     const double s = line_sum<Sh::NT>(res.q.acc, reinterpret_cast<double*>(buf));
     if (threadIdx.x == 0) res.q.part[blockIdx.x] = s;
+  }
+}
+
+template <typename T, int Mh>
+__global__ void __launch_bounds__((RowShape<T, Mh>::NT)) k_residual_rows(RowArgs<T> a, RowResidual<T> res) {
+  using Sh = RowShape<T, Mh>;
+  __shared__ __align__(16) cx<T> buf[Sh::RW * Sh::P < Sh::NT ? Sh::NT : Sh::RW * Sh::P];
+  bind_scalars(res.q);
+  const int j = threadIdx.x % Sh::Plan::nj, l = threadIdx.x / Sh::Plan::nj;
+  const int row = blockIdx.x * Sh::RW + l, rc = min(row, a.nrows - 1);
+  row_residual<T, Mh>(a, res, a.src + (long)rc * (Mh + 1), a.dst + (long)rc * (Mh + 1), rc, j, row < a.nrows,
+                      [&](int i) { return &buf[l * Sh::P + Sh::pad(i)]; }, false);
+  if (res.q.part) {
+    const double s = line_sum<Sh::NT>(res.q.acc, reinterpret_cast<double*>(buf));
+    if (threadIdx.x == 0) res.q.part[blockIdx.x] = s;
+  }
+}
+
+// ---------------------------------------------------------------- planes
+// The inverse y and x passes, the single-resolution residual and the forward
+// x and y passes of one z plane in one workgroup, the plane's region rows in
+// LDS.  The three kernels it stands for take 4 to 5 us each at these sizes,
+// launch and memory latency and little else; one kernel waits once.  A plane
+// is one compute unit's work, so it only pays while that is little: us per
+// update of 25 steps, separate passes and planes, float32: 32x32x32 568 and
+// 381, 64x64x64 626 and 493, 64x128x64 692 and 520, 128x64x64 684 and 570,
+// 128x128x64 732 and 752; float64: 540 and 400, 641 and 586, 701 and 680, 706
+// and 765, 861 and 1175.  Hence the caps on M0 M1.  (The inverse and the
+// forward half by planes around the products with W: no gain.)
+template <typename T> constexpr int plane_cap() { return sizeof(T) == 4 ? 8192 : 4096; }
+constexpr int kPlaneNT = 576;  // 9 wavefronts: 36 lines of 16 threads, 72 of 8
+template <typename T> struct PlaneArgs {
+  const cx<T>* twy;  // length-MY table
+  int n1;            // region rows per plane
+  cx<T>* T1;         // planes of MY rows of Mh + 1, in and out
+  RowArgs<T> x;
+};
+template <typename T, int Mh, int MY> struct PlaneShape {
+  using Plan = LinePlan<MY, 16>;
+  using Row = RowShape<T, Mh>;
+  static constexpr int LY = kPlaneNT / Plan::nj, LX = kPlaneNT / Row::Plan::nj;
+  static constexpr int EY = MY * LY, EX = LX * Row::P;
+  static constexpr int E = EY > EX ? EY : EX;    // exchange buffer
+  static constexpr int rows = MY / 2 + 1;        // region rows a torus of twice the data holds
+  static_assert(E * sizeof(cx<T>) >= kPlaneNT * sizeof(double), "reduction scratch");
+  static_assert((E + rows * (Mh + 1)) * sizeof(cx<T>) <= 160 * 1024, "LDS");
+};
+template <typename T, int Mh, int MY>
+__global__ void __launch_bounds__(kPlaneNT) k_plane(PlaneArgs<T> a, RowResidual<T> res) {
+  using Sh = PlaneShape<T, Mh, MY>;
+  using Plan = typename Sh::Plan;
+  using Row = typename Sh::Row;
+  constexpr int H0 = Mh + 1, R1 = Plan::template radix<false>(0), B1 = MY / R1, RL = Plan::last, BL = MY / RL;
+  __shared__ __align__(16) cx<T> buf[Sh::E];
+  __shared__ __align__(16) cx<T> plane[Sh::rows * H0];
+  bind_scalars(res.q);
+  const int z = blockIdx.x, t = threadIdx.x;
+  cx<T>* P = a.T1 + (long)z * MY * H0;
+  const int b = t % Sh::LY, jy = t / Sh::LY;
+  auto aty = [&](int i) { return &buf[i * Sh::LY + b]; };
+  for (int c0 = 0; c0 < H0; c0 += Sh::LY) {
+    const int c = c0 + b, cc = min(c, H0 - 1);
+    cx<T> v[Plan::rmax];
+    if (jy < B1) {
+#pragma unroll
+      for (int r = 0; r < R1; ++r) v[r] = P[(jy + r * B1) * H0 + cc];
+    }
+    line_fft<T, Plan, MY, true, false, 1>(v, jy, a.twy, aty, c0 > 0);
+    if (jy < BL && c < H0) {
+#pragma unroll
+      for (int r = 0; r < RL; ++r) {
+        const int k = jy + r * BL;
+        if (k < a.n1) plane[k * H0 + c] = v[r];
+      }
+    }
+  }
+  __syncthreads();
+  const int jx = t % Row::Plan::nj, l = t / Row::Plan::nj;
+  auto atx = [&](int i) { return &buf[l * Row::P + Row::pad(i)]; };
+  for (int r0 = 0; r0 < a.n1; r0 += Sh::LX) {
+    const int y = r0 + l, yc = min(y, a.n1 - 1), row = z * a.n1 + yc;
+    cx<T>* X = plane + yc * H0;
+    row_residual<T, Mh>(a.x, res, X, X, row, jx, y < a.n1, atx, true);
+  }
+  __syncthreads();
+  for (int c0 = 0; c0 < H0; c0 += Sh::LY) {
+    const int c = c0 + b, cc = min(c, H0 - 1);
+    cx<T> v[Plan::rmax];
+    if (jy < B1) {
+#pragma unroll
+      for (int r = 0; r < R1; ++r) {
+        const int k = jy + r * B1;
+        v[r] = mk<T>(0, 0);
+        if (r * B1 < a.n1) {  // uniform; rows past the region are zero
+          const cx<T> x = plane[min(k, a.n1 - 1) * H0 + cc];
+          v[r].x = k < a.n1 ? x.x : (T)0;
+          v[r].y = k < a.n1 ? x.y : (T)0;
+        }
+      }
+    }
+    line_fft<T, Plan, MY, false, false, 1>(v, jy, a.twy, aty, true);
+    if (jy < BL && c < H0) {
+#pragma unroll
+      for (int r = 0; r < RL; ++r) P[(jy + r * BL) * H0 + c] = v[r];
+    }
+  }
+  if (res.q.part) {
+    const double s = line_sum<kPlaneNT>(res.q.acc, reinterpret_cast<double*>(buf));
+    if (t == 0) res.q.part[z] = s;
   }
 }
 
@@ -680,7 +790,8 @@ __global__ void __launch_bounds__((StridedShape<double, M>::NT)) k_corr_z(CorrZ 
               hipStream_t s);                                                                                      \
   int rows_c2r(int Mh, const RowArgs<T>& a, hipStream_t s);                                                        \
   int rows_r2c(int Mh, const RowArgs<T>& a, const LoadResidual<T>& res, hipStream_t s);                            \
-  int rows_residual(int Mh, const RowArgs<T>& a, const LoadResidual<T>& res, hipStream_t s);
+  int rows_residual(int Mh, const RowArgs<T>& a, const LoadResidual<T>& res, hipStream_t s);                        \
+  int plane_residual(int Mh, int MY, int nz, const PlaneArgs<T>& a, const LoadResidual<T>& res, hipStream_t s);
 DR_LINE_API(float)
 DR_LINE_API(double)
 #undef DR_LINE_API
