@@ -1827,13 +1827,13 @@ struct Chain : public ChainBase {
       if (prof && L >= 2 && s == L - 1) DR_HIP(hipEventRecord(ev[1], stream));
     }
     // final half kick at B with the energies of the end point
-    EpiMomentum<T> em{muB.p, p.p, invlam.p, spec(), (T)(0.5 * eps), (T)sigma[0], H0, nullptr, nullptr, 1, part.p,
-                      pstride, S_PRIOR_B, S_TMP, S_KIN_B, S_TMP, 0.0, 0.0, 0.0, 0.0, gsc};
-    const int zb = zgrid();
+    EpiMomentum<T> em{muB.p, p.p, invlam.p, spec(), (T)(0.5 * eps), (T)sigma[0], H0, pslot(S_PRIOR_B), pslot(S_KIN_B),
+                      0.0, 0.0, gsc};
+    const int zl = lines_ok(2, P_Z) ? lines_z_kick(M[2], axis_dev<T>(2).tw, M[1] * H0, reg[2], T1.p, em, stream) : 0;
+    const int zb = zl ? zl : zgrid();
     note_blocks(S_PRIOR_B, zb);
     note_blocks(S_KIN_B, zb);
-    note_blocks(S_TMP, zb);
-    strided<T, false>(2, 1, M[1] * H0, reg[2], M[2], LoadS<T>{{}, T1.p, 0, sk}, em);
+    if (!zl) strided<T, false>(2, 1, M[1] * H0, reg[2], M[2], LoadS<T>{{}, T1.p, 0, sk}, em);
     if (compat()) {
       // imaginary chain: all L steps per mode in one pass
       const int g = (int)std::min<long>(cdiv(Ns, kThreads), 4096);

@@ -76,65 +76,6 @@ template <typename T> struct StoreSpec : NoRed {
   __device__ __forceinline__ void store(int, int k, int b, cx<T> v) const { dst[sp.at(k, b)] = v; }
 };
 
-// momentum update p += coef * (F(S r) - mu/lambda) fused into the last
-// forward pass (MultiResParameters.h:690,699 with _compute_gradient :349-374);
-// optional reductions of the prior and kinetic energies (Parseval).
-template <typename T> struct EpiMomentum {
-  const cx<T>* X; cx<T>* p; const T* invlam; Spec<T> sp; T coef; T sig; int H0;
-  const cx<T>* Xi; cx<T>* pim;
-  int do_red; double* part; long pstride; int s_prior, s_priori, s_kin, s_kini;
-  double a0, a1, a2, a3;
-  const StepScalars<T>* sc;  // half kick
-  __device__ __forceinline__ void bind() {
-    if (sc) {
-      coef = sc->half;
-      sig = sc->sig0;
-    }
-  }
-  // the state one mode's update reads (k_strided fetches several modes'
-  // state before updating them)
-  struct State { T il; cx<T> x, p, xi, pi; };
-  __device__ __forceinline__ State fetch(int, int k, int b) const {
-    const long i = sp.at(k, b);
-    State s{invlam[i], X[i], p[i], mk<T>(0, 0), mk<T>(0, 0)};
-    if (pim) {
-      s.xi = Xi[i];
-      s.pi = pim[i];
-    }
-    return s;
-  }
-  __device__ __forceinline__ void store(int o, int k, int b, cx<T> v) { store(o, k, b, v, fetch(o, k, b)); }
-  __device__ __forceinline__ void store(int, int k, int b, cx<T> v, const State& s) {
-    const long i = sp.at(k, b);
-    const T il = s.il;
-    const cx<T> x = s.x;
-    const cx<T> pn = s.p + (v - x * il) * coef;
-    p[i] = pn;
-    cx<T> xi = mk<T>(0, 0), pin = mk<T>(0, 0);
-    if (pim) {
-      xi = s.xi;
-      pin = s.pi - xi * (il * coef);
-      pim[i] = pin;
-    }
-    if (do_red) {
-      const double w = herm_w(b % H0, H0);
-      const double ild = (double)il;
-      const double ilm = il > (T)0 ? 1.0 / (double)(il + sig) : 0.0;
-      a0 += w * ild * ((double)x.x * x.x + (double)x.y * x.y);
-      a2 += w * ilm * ((double)pn.x * pn.x + (double)pn.y * pn.y);
-      a1 += w * ild * ((double)xi.x * xi.x + (double)xi.y * xi.y);
-      a3 += w * ilm * ((double)pin.x * pin.x + (double)pin.y * pin.y);
-    }
-  }
-  __device__ __forceinline__ void finish(double* red, int blk) {
-    if (!do_red) return;
-    red_write(a0, red, part + s_prior * pstride, blk);
-    red_write(a1, red, part + s_priori * pstride, blk);
-    red_write(a2, red, part + s_kin * pstride, blk);
-    red_write(a3, red, part + s_kini * pstride, blk);
-  }
-};
-
 // kick then drift between two gradients (MultiResParameters.h:690-699):
 //   p  += coef (F(S r) - X/lambda)      with the gradient taken at X
 //   X' =  X + eps p / lambda_m          written to Xd and returned for the
@@ -193,6 +134,47 @@ template <typename T> struct MidLeapfrog {
   __device__ __forceinline__ cx<T> apply(int k, int b, cx<T> v) { return apply(k, b, v, fetch(k, b)); }
   __device__ __forceinline__ void finish(double* red, int blk) {
     if (do_red) red_write(a0, red, part, blk);
+  }
+};
+
+// momentum update p += coef * (F(S r) - mu/lambda) fused into the last
+// forward pass (MultiResParameters.h:690,699 with _compute_gradient :349-374)
+// with reductions of the prior and kinetic energies (Parseval).
+template <typename T> struct EpiMomentum {
+  const cx<T>* X; cx<T>* p; const T* invlam; Spec<T> sp; T coef; T sig; int H0;
+  double* part_prior; double* part_kin;
+  double a0, a1;
+  const StepScalars<T>* sc;  // half kick
+  __device__ __forceinline__ void bind() {
+    if (sc) {
+      coef = sc->half;
+      sig = sc->sig0;
+    }
+  }
+  // the state one mode's update reads (several modes' state is fetched before
+  // their updates)
+  struct State { cx<T> x, p; T il; };
+  template <class I> __device__ __forceinline__ State fetch_at(I i) const {
+    return State{nt_ld(X + i), nt_ld(p + i), invlam[i]};
+  }
+  // mode i of column b; write = false leaves memory and the sums alone
+  template <class I> __device__ __forceinline__ void apply_at(I i, int b, cx<T> v, const State& s, bool write) {
+    const cx<T> pn = s.p + (v - s.x * s.il) * coef;
+    if (!write) return;
+    nt_st(p + i, pn);
+    const double w = herm_w(b % H0, H0);
+    const double ilm = s.il > (T)0 ? 1.0 / (double)(s.il + sig) : 0.0;
+    a0 += w * (double)s.il * ((double)s.x.x * s.x.x + (double)s.x.y * s.x.y);
+    a1 += w * ilm * ((double)pn.x * pn.x + (double)pn.y * pn.y);
+  }
+  __device__ __forceinline__ State fetch(int, int k, int b) const { return fetch_at(sp.at(k, b)); }
+  __device__ __forceinline__ void store(int o, int k, int b, cx<T> v) { store(o, k, b, v, fetch(o, k, b)); }
+  __device__ __forceinline__ void store(int, int k, int b, cx<T> v, const State& s) {
+    apply_at(sp.at(k, b), b, v, s, true);
+  }
+  __device__ __forceinline__ void finish(double* red, int blk) {
+    red_write(a0, red, part_prior, blk);
+    red_write(a1, red, part_kin, blk);
   }
 };
 

@@ -26,6 +26,22 @@ int lines_z(int M, const cx<LT>* tw, int nb, int n_in, int n_out, cx<LT>* T1, co
   }
 #undef DR_CASE
 }
+int lines_z_kick(int M, const cx<LT>* tw, int nb, int n_in, const cx<LT>* T1, const EpiMomentum<LT>& em,
+                 hipStream_t s) {
+#define DR_CASE(m)                                                                                       \
+  case m: {                                                                                              \
+    using Sh = ZShape<LT, m>;                                                                            \
+    const int g = cdiv(nb, Sh::TB);                                                                      \
+    hipLaunchKernelGGL((k_zkick<LT, m>), dim3(g), dim3(Sh::NT), 0, s, tw, nb, n_in, T1, em);             \
+    DR_HIP(hipGetLastError());                                                                           \
+    return g;                                                                                            \
+  }
+  switch (M) {
+    DR_LINE_LENGTHS(DR_CASE)
+    default: return 0;
+  }
+#undef DR_CASE
+}
 #elif DR_LINES_PASS == 5
 int lines_corr(int M, const CorrZ& a, hipStream_t s) {
 #define DR_CASE(m)                                                                                       \

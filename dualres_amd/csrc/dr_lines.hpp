@@ -270,6 +270,21 @@ template <typename T> constexpr int line_np(int rl) {
   const int m = 4;
   return rl < m ? rl : m;
 }
+// a column's n_in input rows, the rest zero, for the first stage
+template <typename T, int R1, int B1>
+__device__ __forceinline__ void z_load(cx<T>* v, int j, const cx<T>* src, int nb, int n_in) {
+  if (j >= B1) return;
+#pragma unroll
+  for (int r = 0; r < R1; ++r) {
+    v[r] = mk<T>(0, 0);
+    if (r * B1 < n_in) {  // uniform
+      const int k = j + r * B1;
+      const cx<T> x = src[(unsigned)(min(k, n_in - 1) * nb)];
+      v[r].x = k < n_in ? x.x : (T)0;
+      v[r].y = k < n_in ? x.y : (T)0;
+    }
+  }
+}
 template <typename T, int M>
 __global__ void __launch_bounds__((ZShape<T, M>::NT))
 k_zlines(const cx<T>* tw, int nb, int n_in, int n_out, cx<T>* T1, MidLeapfrog<T> mid) {
@@ -284,18 +299,7 @@ k_zlines(const cx<T>* tw, int nb, int n_in, int n_out, cx<T>* T1, MidLeapfrog<T>
   const bool in = c < nb;
   const int cc = in ? c : nb - 1;
   cx<T> v[Plan::rmax];
-  if (j < B1) {
-#pragma unroll
-    for (int r = 0; r < R1; ++r) {
-      v[r] = mk<T>(0, 0);
-      if (r * B1 < n_in) {
-        const int k = j + r * B1;
-        const cx<T> x = T1[(unsigned)(min(k, n_in - 1) * nb + cc)];
-        v[r].x = k < n_in ? x.x : (T)0;
-        v[r].y = k < n_in ? x.y : (T)0;
-      }
-    }
-  }
+  z_load<T, R1, B1>(v, j, T1 + cc, nb, n_in);
   // mode k of the column in the state's layout
   const unsigned s0 = (unsigned)Spec<T>{M, nb}.at(0, cc);
   auto si = [&](int k) { return s0 + (unsigned)(k * Spec<T>::C); };
@@ -330,6 +334,48 @@ k_zlines(const cx<T>* tw, int nb, int n_in, int n_out, cx<T>* T1, MidLeapfrog<T>
     const double s = line_sum<NT>(in ? mid.a0 : 0.0, reinterpret_cast<double*>(buf));
     if (threadIdx.x == 0) mid.part[blockIdx.x] = s;
   }
+}
+
+// The leapfrog's last half kick: forward transform, p's update and the end
+// point's energies (EpiMomentum), nothing back.  Same shape as the z pass.
+// Once per update: 64x64x32 float32 23 -> 5 us against the tile kernel, 256x512x256
+// float64 251 -> 212 (281 with cached loads of the state behind a branch).
+template <typename T, int M>
+__global__ void __launch_bounds__((ZShape<T, M>::NT))
+k_zkick(const cx<T>* tw, int nb, int n_in, const cx<T>* T1, EpiMomentum<T> em) {
+  using Plan = typename ZShape<T, M>::Plan;
+  constexpr int TB = ZShape<T, M>::TB, R1 = Plan::template radix<false>(0), B1 = M / R1, RL = Plan::last,
+                BL = M / RL, NT = ZShape<T, M>::NT, NP = line_np<T>(RL);
+  __shared__ __align__(16) cx<T> buf[M * TB];
+  bind_scalars(em);
+  const int b = threadIdx.x % TB, j = threadIdx.x / TB;
+  const int c = xcd_tile(blockIdx.x, gridDim.x) * TB + b;
+  const bool in = c < nb;
+  const int cc = in ? c : nb - 1;
+  cx<T> v[Plan::rmax];
+  z_load<T, R1, B1>(v, j, T1 + cc, nb, n_in);
+  const unsigned s0 = (unsigned)Spec<T>{M, nb}.at(0, cc);
+  auto si = [&](int k) { return s0 + (unsigned)(k * Spec<T>::C); };
+  typename EpiMomentum<T>::State st[NP];
+#pragma unroll
+  for (int r = 0; r < NP; ++r) st[r] = em.fetch_at(si(j + r * BL));
+  line_fft<T, Plan, M, false, false, 1>(v, j, tw, [&](int i) { return &buf[i * TB + b]; }, false);
+#pragma unroll
+  for (int r0 = 0; r0 < RL; r0 += NP) {
+    if (r0 > 0) {
+#pragma unroll
+      for (int u = 0; u < NP; ++u)
+        if (r0 + u < RL) st[u] = em.fetch_at(si(j + (r0 + u) * BL));
+    }
+#pragma unroll
+    for (int u = 0; u < NP; ++u)
+      if (r0 + u < RL) em.apply_at(si(j + (r0 + u) * BL), cc, v[r0 + u], st[u], in);
+  }
+  double* sh = reinterpret_cast<double*>(buf);
+  const double prior = line_sum<NT>(em.a0, sh);
+  if (threadIdx.x == 0) em.part_prior[blockIdx.x] = prior;
+  const double kin = line_sum<NT>(em.a1, sh);
+  if (threadIdx.x == 0) em.part_kin[blockIdx.x] = kin;
 }
 
 // ---------------------------------------------------------------- rows along x
@@ -788,6 +834,8 @@ __global__ void __launch_bounds__((StridedShape<double, M>::NT)) k_corr_z(CorrZ 
   int lines_forward(int M, const LineArgs<T>& a, hipStream_t s);                                                   \
   int lines_z(int M, const cx<T>* tw, int nb, int n_in, int n_out, cx<T>* T1, const MidLeapfrog<T>& mid,           \
               hipStream_t s);                                                                                      \
+  int lines_z_kick(int M, const cx<T>* tw, int nb, int n_in, const cx<T>* T1, const EpiMomentum<T>& em,            \
+                   hipStream_t s);                                                                                 \
   int rows_c2r(int Mh, const RowArgs<T>& a, hipStream_t s);                                                        \
   int rows_r2c(int Mh, const RowArgs<T>& a, const LoadResidual<T>& res, hipStream_t s);                            \
   int rows_residual(int Mh, const RowArgs<T>& a, const LoadResidual<T>& res, hipStream_t s);                        \
