@@ -191,7 +191,9 @@ int dr_update_captured(dr_chain* c, double eps, int L, double u_accept, dr_updat
  * device architecture, precision, state mode, dataset count, torus and image
  * region; a timed result is added to that file.  The tile choice changes
  * only the blocking of the energy reductions, the radix order the rounding
- * of the transforms.  dr_set_tuning applies params (-1: built-in rule). */
+ * of the transforms.  dr_set_tuning applies params (-1: built-in rule, the
+ * register line kernels where the length has one; a tile size or a radix order
+ * other than 0 selects the tile kernels for that pass or axis). */
 int dr_autotune(dr_chain* c, const char* cache_path, int* params, int* from_cache);
 int dr_set_tuning(dr_chain* c, const int* params);
 int dr_get_tuning(dr_chain* c, int* params);
