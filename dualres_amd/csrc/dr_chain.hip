@@ -844,13 +844,17 @@ struct Chain : public ChainBase {
         }
       }
       // a row is interior when its stencil stays inside the region grid on
-      // every axis (then flat offsets and 3D displacements agree)
+      // every axis (then flat offsets and 3D displacements agree) and it is
+      // the first one at its base: the base is its slot of the lattice grid
+      // (coarse voxels that map to one fine voxel have the same row)
+      std::vector<char> taken(nreg, 0);
       for (long i = 0; i < n_s; ++i) {
         if (rcls[i] != cs) continue;
         xyz(rg0[i], b);
         bool ok = true;
         for (int a = 0; a < 3; ++a) ok = ok && b[a] + dmin[a] >= 0 && b[a] + dmax[a] < reg[a];
-        interior[i] = ok;
+        interior[i] = ok && !taken[rg0[i]];
+        if (ok) taken[rg0[i]] = 1;
       }
     }
     std::vector<int32_t> irow, ibase;
