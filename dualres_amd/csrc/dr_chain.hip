@@ -950,7 +950,7 @@ struct Chain : public ChainBase {
         } else {
           idx = it->second;
         }
-        ww[4 * (size_t)idx + (size_t)(a4 - 4 * wdw)] = wD[e];
+        ww[4 * (size_t)idx + (size_t)(a4 - 4 * wdw)] += wD[e];  // a row may name a column twice
       }
       wstart[p + 1] = (int32_t)woff.size();
     }
@@ -1036,7 +1036,7 @@ struct Chain : public ChainBase {
         if (!sx) break;
         const size_t w0 = lm.w.size();
         lm.w.resize(w0 + 4 * lm.nc, (T)0);
-        for (int e : kv.second.e) lm.w[w0 + (size_t)(d3[3 * e] - kv.second.lo)] = wD[e];
+        for (int e : kv.second.e) lm.w[w0 + (size_t)(d3[3 * e] - kv.second.lo)] += wD[e];
         lm.off.push_back((int32_t)(kv.second.lo + R0 * kv.first.second + R01 * kv.first.first));
       }
     }
@@ -1097,7 +1097,7 @@ struct Chain : public ChainBase {
             const size_t w0 = lt.w.size();
             lt.w.resize(w0 + 4 * sx * lt.nc, (T)0);
             for (int e : kv.second.e)
-              lt.w[w0 + (size_t)(sx * (-fdiv(d3[3 * e], sx) - kv.second.lo) + fmod_(d3[3 * e], sx))] = wD[e];
+              lt.w[w0 + (size_t)(sx * (-fdiv(d3[3 * e], sx) - kv.second.lo) + fmod_(d3[3 * e], sx))] += wD[e];
             lt.off.push_back((int32_t)(kv.second.lo + L[0] * (kv.first.second + L[1] * kv.first.first)));
           }
           lt_start.push_back((int32_t)lt.off.size());

@@ -1,6 +1,8 @@
 """W with what a CSR matrix may repeat, in the stencil layout against plain
 CSR: rows with the same entries (several coarse voxels that map to one fine
-voxel), on both sides of the size from which W mu goes by stencil lines."""
+voxel) and columns named twice in a row (a neighbourhood wider than the image
+wraps onto itself), on both sides of the size from which W mu goes by stencil
+lines."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -33,3 +35,18 @@ def test_repeated_rows_match_csr(dims, step, reach, share, copies, precision):
     rng = np.random.default_rng(11)
     at = np.repeat(np.arange(W.shape[0]), np.where(rng.random(W.shape[0]) < share, copies, 1))
     _compare(ijk, W[at], Yh, rng.standard_normal(len(at)), precision)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("dims,step,reach", [
+    ((19, 14, 13), (2, 2, 2), (1, 2, 1)),
+    ((36, 20, 18), (5, 2, 2), (3, 2, 2)),   # the window table and tiles
+    ((127, 61, 30), (2, 1, 2), (3, 2, 1)),  # W mu by lines
+])
+def test_repeated_columns_match_csr(dims, step, reach, precision):
+    """Every entry in two parts, as two entries of one column."""
+    ijk, W, Yh, Ys = _problem(dims, step, reach)
+    parts = np.stack([0.25 * W.data, 0.75 * W.data], axis=1).ravel()
+    W2 = sp.csr_matrix((parts, np.repeat(W.indices, 2), 2 * W.indptr), shape=W.shape)
+    assert W2.nnz == 2 * W.nnz
+    _compare(ijk, W2, Yh, Ys, precision)
