@@ -2590,8 +2590,11 @@ static void write_tune_cache(const std::string& path, const std::map<std::string
   }
   DR_REQUIRE(std::rename(tmp.c_str(), path.c_str()) == 0, DR_ERUNTIME, "autotune: cannot replace the cache " + path);
 }
-// cache key: device architecture, precision, state mode, datasets, torus
-// and image region
+// cache key: device architecture, precision, state mode, datasets, torus and
+// image region, and the set of kernels the choice was timed against: raised
+// whenever a pass gets a kernel that "no tile size" (-1) selects, so that a
+// choice timed without it is timed again (2: the register lines)
+constexpr int kTuneKernels = 2;
 static std::string tune_key(const drh::ChainBase& c) {
   hipDeviceProp_t prop;
   DR_HIP(hipGetDeviceProperties(&prop, c.cfg.device));
@@ -2600,7 +2603,7 @@ static std::string tune_key(const drh::ChainBase& c) {
   std::ostringstream k;
   k << arch << "|" << (c.cfg.precision == DR_FP64 ? "fp64" : "fp32") << "|"
     << (c.cfg.state_mode == DR_STATE_COMPAT ? "compat" : "real") << "|" << c.cfg.n_datasets << "|" << c.M[0] << "x"
-    << c.M[1] << "x" << c.M[2] << "|" << c.reg[0] << "x" << c.reg[1] << "x" << c.reg[2];
+    << c.M[1] << "x" << c.M[2] << "|" << c.reg[0] << "x" << c.reg[1] << "x" << c.reg[2] << "|k" << kTuneKernels;
   return k.str();
 }
 

@@ -188,8 +188,9 @@ int dr_update_captured(dr_chain* c, double eps, int L, double u_accept, dr_updat
  * pipeline keep theirs).  dr_autotune times each choice on the chain's own
  * buffers (a 2-step leapfrog from the current state, which it leaves as it
  * was), unless cache_path names a JSON file that holds an entry for this
- * device architecture, precision, state mode, dataset count, torus and image
- * region; a timed result is added to that file.  The tile choice changes
+ * device architecture, precision, state mode, dataset count, torus, image
+ * region and set of kernels; a timed result is added to that file.  Entries
+ * timed against an earlier set of kernels stay in it and are not used.  The tile choice changes
  * only the blocking of the energy reductions, the radix order the rounding
  * of the transforms.  dr_set_tuning applies params (-1: built-in rule, the
  * register line kernels where the length has one; a tile size or a radix order
