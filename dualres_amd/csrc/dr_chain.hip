@@ -2073,8 +2073,11 @@ struct Chain : public ChainBase {
     }
     return best;
   }
-  // coordinate search: each pass's tile lines over every size the tile and
-  // LDS allow, then each axis's radix order where the runtime stages run
+  // coordinate search from the built-in choice (-1, order 0: the register lines
+  // where the length has one), or from what is set now where that is faster:
+  // each pass's tile lines over every size the tile and LDS allow and back to
+  // the built-in choice, then each axis's radix order where the runtime stages
+  // run
   void autotune(int* prm) override {
     DR_REQUIRE(data_set, DR_ELOGIC, "autotune: data not set");
     const bool prof0 = prof;
@@ -2087,11 +2090,22 @@ struct Chain : public ChainBase {
     const int capy = pick_tbs(M[1], M[1], sizeof(cx<T>), false, 1 << 20, kTileStrided);
     const int capx = pick_tbs(Mh, Mh + 1, sizeof(cx<T>), true, 1 << 20, kTileX);
     const int cap[NPASS] = {capz, capy, capx, capx, capy};
-    set_tuning(cur);
     double best = time_leapfrog();
+    int built_in[NPASS + 3];
+    std::fill(built_in, built_in + NPASS, -1);
+    std::fill(built_in + NPASS, built_in + NPASS + 3, 0);
+    if (!std::equal(cur, cur + NPASS + 3, built_in)) {
+      set_tuning(built_in);
+      const double t = time_leapfrog();
+      if (t <= best) {
+        best = t;
+        std::copy(built_in, built_in + NPASS + 3, cur);
+      }
+    }
     for (int pid = 0; pid < NPASS; ++pid) {
       int arg = cur[pid];
-      for (int v = 0; v <= cap[pid]; ++v) {
+      for (int v = -1; v <= cap[pid]; ++v) {
+        if (v == arg) continue;
         cur[pid] = v;
         set_tuning(cur);
         const double t = time_leapfrog();

@@ -34,3 +34,13 @@ def test_entries_of_the_tile_kernels_are_not_taken(tmp_path):
     entries = json.loads(other.read_text())
     assert entries[old] == TILES and entries[key] == prm  # kept for an engine that still reads it
     c.close()
+
+
+def test_a_search_from_hand_set_tiles_reaches_the_lines():
+    """Two-line tiles are several times slower than the lines on this torus, so
+    a search that can pick the lines does."""
+    c = _chain()
+    c.set_tuning(TILES)
+    prm, _ = c.autotune()
+    assert prm[0] == -1 and c.tuning() == prm
+    c.close()
