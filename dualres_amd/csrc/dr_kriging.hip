@@ -42,6 +42,7 @@
 #include <vector>
 
 #include "dr_common.hpp"
+#include "dr_reduce.hpp"
 
 namespace drh {
 
@@ -756,22 +757,16 @@ __global__ void __launch_bounds__(256) k_clear_absent(const ExtDesc* __restrict_
   for (int i = threadIdx.x; i < d.m; i += 256) w[dlist[d.dl + i]] = 0.0;
 }
 
-// largest diagonal entry of B (one workgroup): 1 / the smallest variance of an
-// offset given all others
+// largest diagonal entry of B (one workgroup), NaN if any is: 1 / the smallest
+// variance of an offset given all others
 __global__ void __launch_bounds__(256) k_max_diag(const double* __restrict__ B, int n, int ld, double* __restrict__ out) {
   __shared__ double m[256];
   double v = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) {
-    const double b = B[(long)i * ld + i];
-    v = b <= v ? v : b;  // a NaN is kept
-  }
+  for (int i = threadIdx.x; i < n; i += 256) v = max_nan(v, B[(long)i * ld + i]);
   m[threadIdx.x] = v;
   __syncthreads();
   for (int st = 128; st > 0; st >>= 1) {
-    if ((int)threadIdx.x < st) {
-      const double o = m[threadIdx.x + st];
-      if (!(o <= m[threadIdx.x])) m[threadIdx.x] = o;
-    }
+    if ((int)threadIdx.x < st) m[threadIdx.x] = max_nan(m[threadIdx.x], m[threadIdx.x + st]);
     __syncthreads();
   }
   if (threadIdx.x == 0) out[0] = m[0];
