@@ -17,8 +17,8 @@
 //     |S| < |D| is solved directly.  At 1 mm (balls of 1,357, rows at the
 //     mask's edge lose up to half of theirs) this is a few per cent of the
 //     direct factorisations' work.
-//     The batches, sorted by size and padded with an identity block to a
-//     multiple of 64, are factorised by a blocked left-looking
+//     The batches, sorted by size and padded with an identity block to the
+//     multiple of 64 of their largest system, are factorised by a blocked left-looking
 //     float64 Cholesky over 64x64 tiles, two launches per tile
 //     column: k_chol_diag subtracts the finished columns' products from the
 //     diagonal tile, factors it and inverts the factor; k_chol_panel does
@@ -1164,6 +1164,7 @@ struct DBuf {
 struct KrigingCSR {
   long nrow = 0, ncol = 0, n_unique = 0, nnz = 0;
   long n_lu = 0;  // unique systems solved by the pivoted LU (Cholesky failed)
+  long n_batches = 0;  // batches of systems factorised directly, Cholesky and LU
   std::vector<int64_t> rp;
   DBuf<int32_t> cols;
   DBuf<double> vals;
@@ -1405,11 +1406,21 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
   d_mx.down(&bmax_diag, 1, s);
   DR_HIP(hipStreamSynchronize(s));
   const bool via_inverse = !kfail && bmax_diag <= 1e4;
-  // Batches of equal padded size, largest first.
+  // Batches, largest systems first.  A batch is a chain of launches per tile
+  // column, and fewer than two workgroups per compute unit leave that chain's
+  // latency in the open, so a batch takes smaller systems (padded to its size)
+  // up to 512 and is cut at a change of padded size only beyond that.  ms with
+  // batches of one size / at least 64 / 256 / 512 / 1,024 systems, indefinite
+  // kernels by LU: 64 systems of a ball of 1,357 141 / 39 / 39 / 39 / 39, 638 406
+  // / 292 / 179 / 200 / 199, 2,353 710 / 709 / 610 / 589 / 591, 1,728 of a ball of
+  // 305 20.2 / 19.3 / 18.8 / 17.7 / 19.1; by Cholesky 638 of 1,357 52 / 37 / 24 /
+  // 25 / 25, 1,728 63 / 62 / 53 / 47 / 51.
+  constexpr int kBatchMin = 512;
   const double budget = 6.0e9;  // bytes of factor scratch per batch
   DBuf<double> d_A, d_b;
   DBuf<SysDesc> d_sd;
   size_t capA = 0, capB = 0, capS = 0;
+  long n_batches = 0;
   // systems (unique indices) solved directly; returns those whose Cholesky failed
   auto solve_all = [&](std::vector<int> uids, bool lu) {
     std::stable_sort(uids.begin(), uids.end(), [&](int a, int b) { return cnt[urow[a]] > cnt[urow[b]]; });
@@ -1421,11 +1432,13 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
       const int bmax = (int)std::max<long>(1, std::min<long>(16384, (long)(budget / per)));
       std::vector<SysDesc> sd;
       const size_t first = pos;
-      while (pos < uids.size() && (int)sd.size() < bmax && cdiv(cnt[urow[uids[pos]]], NB) * NB == np) {
+      while (pos < uids.size() && (int)sd.size() < bmax &&
+             ((int)sd.size() < kBatchMin || cdiv(cnt[urow[uids[pos]]], NB) * NB == np)) {
         const int u = uids[pos++];
         sd.push_back(SysDesc{rp[urow[u]], cnt[urow[u]], usol[u]});
       }
       const int B = (int)sd.size();
+      ++n_batches;
       if ((size_t)B * np * np > capA) { capA = (size_t)B * np * np; d_A.alloc(capA); }
       if ((size_t)B * np > capB) { capB = (size_t)B * np; d_b.alloc(capB); }
       if ((size_t)B > capS) { capS = B; d_sd.alloc(capS); d_fail.alloc(capS); }
@@ -1573,6 +1586,7 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
   out.ncol = nnz_hr;
   out.n_unique = nU;
   out.n_lu = (long)indefinite.size();
+  out.n_batches = n_batches;
   out.rp.assign(n_rows + 1, 0);
   long dropped = 0;
   for (int i = 0; i < n_rows; ++i) {
@@ -1631,6 +1645,13 @@ int dr_csr_solver_counts(dr_csr* m, int64_t* n_cholesky, int64_t* n_lu) {
     DR_REQUIRE(m && n_cholesky && n_lu, DR_ELOGIC, "dr_csr_solver_counts: null argument");
     *n_lu = m->m.n_lu;
     *n_cholesky = m->m.n_unique - m->m.n_lu;
+  });
+}
+
+int dr_csr_routes(dr_csr* m, int64_t* routes) {
+  return drh::guarded([&] {
+    DR_REQUIRE(m && routes, DR_ELOGIC, "dr_csr_routes: null argument");
+    routes[0] = m->m.n_batches;
   });
 }
 

@@ -270,6 +270,10 @@ int dr_csr_copy(dr_csr* m, int64_t* rowptr, int32_t* cols, double* vals);
  * reference, whose colPivHouseholderQr takes every system
  * (kriging_matrix.h:309-313); a diagnostic of which solver ran. */
 int dr_csr_solver_counts(dr_csr* m, int64_t* n_cholesky, int64_t* n_lu);
+/* How the systems were worked on: routes[0] = batches factorised directly, by
+ * Cholesky and by LU.  routes must hold 1 entry.  A diagnostic, no counterpart in
+ * the reference. */
+int dr_csr_routes(dr_csr* m, int64_t* routes);
 int dr_csr_free(dr_csr* m);
 
 /* --- minimum contrast summary (estimate_kernel_parameters.h:53-101) ------- */
