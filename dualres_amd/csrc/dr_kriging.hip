@@ -14,9 +14,10 @@
 //     one of |S|; a refinement step (the residual on S in twice the precision,
 //     the same solve again) leaves the result more accurate than the direct
 //     solve.  A system with
-//     |S| < |D| is solved directly.  At 1 mm (balls of 1,357, rows at the
-//     mask's edge lose up to half of theirs) this is a few per cent of the
-//     direct factorisations' work.
+//     |S| < |D| is solved directly, and so are all where that is the less
+//     work: few systems, or small ones against the ball.  At 1 mm (balls of
+//     1,357, rows at the mask's edge lose up to half of theirs) the inverse's
+//     way is a few per cent of the direct factorisations' work.
 //     The batches, sorted by size and padded with an identity block to the
 //     multiple of 64 of their largest system, are factorised by a blocked left-looking
 //     float64 Cholesky over 64x64 tiles, two launches per tile
@@ -27,7 +28,8 @@
 //     with those inverses (k_solve_chol), then
 //     normalised by their sum (kriging_matrix.h:318-321).  If the Cholesky
 //     of K itself meets a nonpositive pivot (K with its unit diagonal is
-//     indefinite when tau^2 > 1), every system is solved directly, and those
+//     indefinite when tau^2 > 1) or K is ill conditioned, every system is
+//     solved directly, and those
 //     whose Cholesky fails too by a blocked LU with partial pivoting
 //     (k_getrf_panel / k_trsm_lu / k_gemm_lu_mfma, k_solve_lu).
 //  4. Rows gather their system's weights; rows whose weights sum to NaN stay
@@ -499,7 +501,7 @@ __global__ void __launch_bounds__(256) k_chol_panel(double* A, int np, int j) {
 // ---------------------------------------------------------------- K and its inverse
 // K of the ball (kriging_matrix.h:111-138): unit diagonal, float rounding of
 // the kernel at the separately rounded float distance; Kd the same in float64
-// padded with the identity to ld
+// padded with the identity to ld, where asked for
 __global__ void k_kernel_matrix(Geo g, const float* __restrict__ X, int ld, float* __restrict__ K,
                                 double* __restrict__ Kd) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
@@ -517,7 +519,7 @@ __global__ void k_kernel_matrix(Geo g, const float* __restrict__ X, int ld, floa
     }
     K[(long)i * g.nP + j] = (float)v;
   }
-  Kd[(long)i * ld + j] = v;
+  if (Kd) Kd[(long)i * ld + j] = v;
 }
 
 // Wt[c][i] = (L^-1)[i][c]^T from the factor and the inverses of its diagonal
@@ -711,9 +713,16 @@ __global__ void __launch_bounds__(256) k_extend(const ExtDesc* __restrict__ ed, 
 // two-sum; ten operations per entry.  kResRows rows share a thread's K.
 // At 1 mm (4,227 rows of 1,357) 3 ms, as a product on the matrix cores 0.4.
 constexpr int kResRows = 8;
+// sum + low -= w k, low taking what the product and the addition round off
+__device__ __forceinline__ void sub_mul_2(double w, double k, double& sum, double& low) {
+#pragma clang fp contract(off)
+  const double m = -w, q = m * k, qe = __builtin_fma(m, k, -q);
+  const double t = sum + q, v = t - sum;
+  low += ((sum - (t - v)) + (q - v)) + qe;
+  sum = t;
+}
 __global__ void __launch_bounds__(256) k_residual_ext(int E, int ld, const double* __restrict__ Kd,
                                                       const double* __restrict__ W, double* R) {
-#pragma clang fp contract(off)
   __shared__ double sw[kResRows][NB];
   const int j = blockIdx.x * 256 + threadIdx.x, r0 = blockIdx.y * kResRows;
   const int jc = min(j, ld - 1);
@@ -735,12 +744,7 @@ __global__ void __launch_bounds__(256) k_residual_ext(int E, int ld, const doubl
 #pragma unroll
       for (int u = 0; u < 8; ++u)
 #pragma unroll
-        for (int r = 0; r < kResRows; ++r) {
-          const double w = -sw[r][i + u], q = w * k[u], qe = __builtin_fma(w, k[u], -q);
-          const double t = sum[r] + q, v = t - sum[r];
-          low[r] += ((sum[r] - (t - v)) + (q - v)) + qe;
-          sum[r] = t;
-        }
+        for (int r = 0; r < kResRows; ++r) sub_mul_2(sw[r][i + u], k[u], sum[r], low[r]);
     }
   }
   if (j >= ld) return;
@@ -758,11 +762,16 @@ __global__ void __launch_bounds__(256) k_clear_absent(const ExtDesc* __restrict_
 }
 
 // largest diagonal entry of B (one workgroup), NaN if any is: 1 / the smallest
-// variance of an offset given all others
-__global__ void __launch_bounds__(256) k_max_diag(const double* __restrict__ B, int n, int ld, double* __restrict__ out) {
+// variance of an offset given all others.  factor: of 1 / B_ii^2 for a factor B,
+// the same given those before it.
+__global__ void __launch_bounds__(256) k_max_diag(const double* __restrict__ B, int n, int ld, int factor,
+                                                  double* __restrict__ out) {
   __shared__ double m[256];
   double v = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) v = max_nan(v, B[(long)i * ld + i]);
+  for (int i = threadIdx.x; i < n; i += 256) {
+    const double b = B[(long)i * ld + i];
+    v = max_nan(v, factor ? 1.0 / (b * b) : b);
+  }
   m[threadIdx.x] = v;
   __syncthreads();
   for (int st = 128; st > 0; st >>= 1) {
@@ -1014,17 +1023,57 @@ __device__ __forceinline__ void chol_solve(const double* As, int np, int n, doub
   }
 }
 
+// First pass: the solution of each system to sol.  Second pass, bv now the
+// residual: its solution added, normalised to weights.
 __global__ void __launch_bounds__(256) k_solve_chol(const double* A, int np, const SysDesc* __restrict__ sd,
-                                                    const double* __restrict__ bv, double* __restrict__ sol) {
+                                                    const double* __restrict__ bv, double* __restrict__ sol,
+                                                    int second) {
   extern __shared__ double y[];
   __shared__ double part[4][NB];
   __shared__ double rk[NB];
   const int s = blockIdx.x;
   const SysDesc d = sd[s];
+  double* x = sol + d.sol;
   for (int i = threadIdx.x; i < np; i += 256) y[i] = bv[(long)s * np + i];
   __syncthreads();
   chol_solve(A + (long)s * np * np, np, d.n, y, part, rk);
-  normalise_out(y, d.n, &part[0][0], sol + d.sol);
+  if (!second) {
+    for (int i = threadIdx.x; i < d.n; i += 256) x[i] = y[i];
+    return;
+  }
+  for (int i = threadIdx.x; i < d.n; i += 256) y[i] += x[i];
+  __syncthreads();
+  normalise_out(y, d.n, &part[0][0], x);
+}
+
+// bv -= K[S, S] sol in twice the precision, for systems solved directly (as
+// k_residual_ext): 64 rows of system blockIdx.x per workgroup, each wavefront a
+// quarter of the columns.  K is symmetric, so the lanes read along its rows.
+__global__ void __launch_bounds__(256) k_residual_sys(const SysDesc* __restrict__ sd, const float* __restrict__ K,
+                                                      int nP, const int* __restrict__ pidx, int np,
+                                                      const double* __restrict__ sol, double* __restrict__ bv) {
+  __shared__ double ps[4][64], pl[4][64];
+  const SysDesc d = sd[blockIdx.x];
+  const int r0 = blockIdx.y * 64;
+  if (r0 >= d.n) return;
+  const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int* id = pidx + d.off;
+  const double* x = sol + d.sol;
+  const int i = min(r0 + lane, d.n - 1), c = id[i];
+  double* b = bv + (long)blockIdx.x * np + i;
+  double sum = q == 0 ? *b : 0.0, low = 0.0;
+  const int j1 = (int)((long)d.n * (q + 1) / 4);
+#pragma unroll 4
+  for (int j = (int)((long)d.n * q / 4); j < j1; ++j) sub_mul_2(x[j], (double)K[(long)id[j] * nP + c], sum, low);
+  ps[q][lane] = sum;
+  pl[q][lane] = low;
+  __syncthreads();
+  if (q > 0 || r0 + lane >= d.n) return;
+  for (int k = 1; k < 4; ++k) {
+    sub_mul_2(-1.0, ps[k][lane], sum, low);
+    low += pl[k][lane];
+  }
+  *b = sum + low;
 }
 
 // y on the absent offsets of an extended system with F B in U, to its row of
@@ -1165,6 +1214,8 @@ struct KrigingCSR {
   long nrow = 0, ncol = 0, n_unique = 0, nnz = 0;
   long n_lu = 0;  // unique systems solved by the pivoted LU (Cholesky failed)
   long n_batches = 0;  // batches of systems factorised directly, Cholesky and LU
+  bool inverse_built = false;  // K^-1 was computed
+  long n_inverse = 0;          // unique systems solved through it
   std::vector<int64_t> rp;
   DBuf<int32_t> cols;
   DBuf<double> vals;
@@ -1368,16 +1419,34 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
   long solsz = 0;
   for (int u = 0; u < nU; ++u) { usol[u] = solsz; solsz += cnt[urow[u]]; }
   DBuf<double> d_sol(solsz);
-  // K, its factor and its inverse
+  // Which way: directly a system's Cholesky is n^3 / 3 operations and its
+  // refinement's residual 10 n^2.  Through the inverse it is a Cholesky of the
+  // smaller of n and m = nP - n and, where that is m, four products with B and
+  // the residual, 18 nP^2.  The inverse itself is nP^3 (K's factor, the factor's
+  // inverse and their product, a third each), but as a chain of launches with
+  // few workgroups: at a twelfth of the batches' rate.  ms through the inverse
+  // and directly, with operations so counted, inverse / direct, in brackets.
+  // 57 offsets: never below 1.2, directly 0.2 to 0.4 ms sooner.  123: 64 systems
+  // 0.90, 0.64 [2.1]; 413 1.11, 0.83 [0.84]; 1,728 2.1, 2.4 [0.76].  305: 47 1.5,
+  // 1.0 [1.8]; 82 1.5, 1.5 [2.3]; 210 1.6, 1.9 [0.92]; 1,728 3.5, 5.5 [0.42].
+  // 1,357: 64 8.4, 5.5 [2.0]; 210 10.8, 8.0 [1.1]; 197 of more offsets 17, 20
+  // [0.52]; 1,728 19, 47 [0.22].  4,729: 64 87, 31 [4.8]; 210 143, 66 [2.3]; 672
+  // 225, 318 [0.82]; 1,728 314, 1,351 [0.22].
   const int ld = cdiv(nP, NB) * NB, ntl = ld / NB;
+  double ops_direct = 0.0, ops_inverse = 12.0 * std::pow((double)nP, 3);
+  for (int u = 0; u < nU; ++u) {
+    const double n = cnt[urow[u]], m = std::min<double>(n, nP - n);
+    ops_direct += n * n * n / 3 + 10 * n * n;
+    ops_inverse += m * m * m / 3 + (m < n ? 18.0 * nP * nP : 0.0);
+  }
+  bool via_inverse = ops_inverse < ops_direct;
   DBuf<float> d_X(X.size()), d_K((size_t)nP * nP);
-  DBuf<double> d_Kd((size_t)ld * ld), d_L((size_t)ld * ld);
+  DBuf<double> d_Kd, d_B;
   DBuf<int> d_fail(1);
+  if (via_inverse) d_Kd.alloc((size_t)ld * ld);
   d_X.up(X.data(), X.size(), s);
   hipLaunchKernelGGL(k_kernel_matrix, dim3(cdiv(ld, 256), ld), dim3(256), 0, s, g, d_X.p, ld, d_K.p, d_Kd.p);
   DR_HIP(hipGetLastError());
-  DR_HIP(hipMemcpyAsync(d_L.p, d_Kd.p, (size_t)ld * ld * sizeof(double), hipMemcpyDeviceToDevice, s));
-  DR_HIP(hipMemsetAsync(d_fail.p, 0, sizeof(int), s));
   auto cholesky = [&](double* A, int B, int np) {
     const int nt = np / NB;
     for (int k = 0; k < nt; ++k) {
@@ -1386,26 +1455,39 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
       DR_HIP(hipGetLastError());
     }
   };
-  cholesky(d_L.p, 1, ld);
-  // K^-1 = (L^-1)^T L^-1 into d_B.  Systems go through it only where K is
-  // well conditioned: a diagonal entry of K^-1 above 1e4 (a variance given
-  // all others below 1e-4; it is at least 1 - tau^2) keeps the direct solves.
-  DBuf<double> d_B((size_t)ld * ld), d_mx(1);
-  {
-    DBuf<double> d_Wt((size_t)ld * ld);
-    hipLaunchKernelGGL(k_tri_inverse, dim3(ntl, NB / 16), dim3(256), 0, s, d_L.p, ld, d_Wt.p);
-    hipLaunchKernelGGL(k_gemm_xyt, dim3(ntl, ntl), dim3(256), 0, s, d_Wt.p, d_Wt.p, ld, ntl, 1,
-                       (const double*)nullptr, d_B.p);
-    hipLaunchKernelGGL(k_max_diag, dim3(1), dim3(256), 0, s, d_B.p, nP, ld, d_mx.p);
-    DR_HIP(hipGetLastError());
-    DR_HIP(hipStreamSynchronize(s));
+  // K's factor and K^-1 = (L^-1)^T L^-1 into d_B.  Systems go through it only
+  // where K is positive definite and well conditioned: a diagonal entry of K^-1
+  // above 1e4 (a variance given all others below 1e-4; it is at least
+  // 1 - tau^2) keeps the direct solves.  1 / L_ii^2 is no larger than that
+  // entry, so most such K are known from the factor, before the inverse.
+  bool inverse_built = false;
+  if (via_inverse) {
+    DBuf<double> d_L((size_t)ld * ld), d_mx(1);
+    DR_HIP(hipMemcpyAsync(d_L.p, d_Kd.p, (size_t)ld * ld * sizeof(double), hipMemcpyDeviceToDevice, s));
+    DR_HIP(hipMemsetAsync(d_fail.p, 0, sizeof(int), s));
+    cholesky(d_L.p, 1, ld);
+    auto within = [&](const double* A, int factor) {
+      int kfail = 0;
+      double mx = 0.0;
+      hipLaunchKernelGGL(k_max_diag, dim3(1), dim3(256), 0, s, A, nP, ld, factor, d_mx.p);
+      DR_HIP(hipGetLastError());
+      d_fail.down(&kfail, 1, s);
+      d_mx.down(&mx, 1, s);
+      DR_HIP(hipStreamSynchronize(s));
+      return !kfail && mx <= 1e4;
+    };
+    via_inverse = within(d_L.p, 1);
+    if (via_inverse) {
+      DBuf<double> d_Wt((size_t)ld * ld);
+      d_B.alloc((size_t)ld * ld);
+      hipLaunchKernelGGL(k_tri_inverse, dim3(ntl, NB / 16), dim3(256), 0, s, d_L.p, ld, d_Wt.p);
+      hipLaunchKernelGGL(k_gemm_xyt, dim3(ntl, ntl), dim3(256), 0, s, d_Wt.p, d_Wt.p, ld, ntl, 1,
+                         (const double*)nullptr, d_B.p);
+      DR_HIP(hipGetLastError());
+      inverse_built = true;
+      via_inverse = within(d_B.p, 0);  // waits: the factor and Wt are freed here
+    }
   }
-  int kfail = 0;
-  double bmax_diag = 0.0;
-  d_fail.down(&kfail, 1, s);
-  d_mx.down(&bmax_diag, 1, s);
-  DR_HIP(hipStreamSynchronize(s));
-  const bool via_inverse = !kfail && bmax_diag <= 1e4;
   // Batches, largest systems first.  A batch is a chain of launches per tile
   // column, and fewer than two workgroups per compute unit leave that chain's
   // latency in the open, so a batch takes smaller systems (padded to its size)
@@ -1463,8 +1545,13 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
                            d_fail.p, d_sol.p);
       } else {
         cholesky(d_A.p, B, np);
-        hipLaunchKernelGGL(k_solve_chol, dim3(B), dim3(256), np * sizeof(double), s, d_A.p, np, d_sd.p, d_b.p,
-                           d_sol.p);
+        for (int second = 0; second < 2; ++second) {  // refined once, as the extended systems are
+          if (second)
+            hipLaunchKernelGGL(k_residual_sys, dim3(B, nt), dim3(256), 0, s, d_sd.p, d_K.p, nP, d_pidx.p, np, d_sol.p,
+                               d_b.p);
+          hipLaunchKernelGGL(k_solve_chol, dim3(B), dim3(256), np * sizeof(double), s, d_A.p, np, d_sd.p, d_b.p,
+                             d_sol.p, second);
+        }
       }
       DR_HIP(hipGetLastError());
       std::vector<int> fail(B);
@@ -1483,6 +1570,7 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
   // Slabs of bounded factor and row memory, the largest factorisations first.
   auto msize = [&](int u) { return std::min(cnt[urow[u]], nP - cnt[urow[u]]); };
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return msize(a) > msize(b); });
+  long n_inverse = 0;
   for (size_t e0 = 0; e0 < order.size();) {
     std::vector<ExtDesc> ed;
     std::vector<FacDesc> fd;
@@ -1561,8 +1649,12 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
     std::vector<int> ef(nf);
     if (nf) d_ef.down(ef.data(), nf, s);
     DR_HIP(hipStreamSynchronize(s));
+    n_inverse += E;
     for (int i = 0; i < nf; ++i)
-      if (ef[i]) direct.push_back(fu[i]);  // again on its own, and by LU if that fails too
+      if (ef[i]) {
+        direct.push_back(fu[i]);  // again on its own, and by LU if that fails too
+        n_inverse -= fd[i].row >= 0;
+      }
   }
   const std::vector<int> indefinite = solve_all(direct, false);
   if (!indefinite.empty()) (void)solve_all(indefinite, true);
@@ -1587,6 +1679,8 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
   out.n_unique = nU;
   out.n_lu = (long)indefinite.size();
   out.n_batches = n_batches;
+  out.inverse_built = inverse_built;
+  out.n_inverse = n_inverse;
   out.rp.assign(n_rows + 1, 0);
   long dropped = 0;
   for (int i = 0; i < n_rows; ++i) {
@@ -1652,6 +1746,8 @@ int dr_csr_routes(dr_csr* m, int64_t* routes) {
   return drh::guarded([&] {
     DR_REQUIRE(m && routes, DR_ELOGIC, "dr_csr_routes: null argument");
     routes[0] = m->m.n_batches;
+    routes[1] = m->m.inverse_built ? 1 : 0;
+    routes[2] = m->m.n_inverse;
   });
 }
 

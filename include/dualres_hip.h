@@ -271,8 +271,10 @@ int dr_csr_copy(dr_csr* m, int64_t* rowptr, int32_t* cols, double* vals);
  * (kriging_matrix.h:309-313); a diagnostic of which solver ran. */
 int dr_csr_solver_counts(dr_csr* m, int64_t* n_cholesky, int64_t* n_lu);
 /* How the systems were worked on: routes[0] = batches factorised directly, by
- * Cholesky and by LU.  routes must hold 1 entry.  A diagnostic, no counterpart in
- * the reference. */
+ * Cholesky and by LU; [1] whether the inverse of the whole neighbourhood's kernel
+ * matrix was computed; [2] the unique systems solved through it (0 although it
+ * was computed: it was too ill conditioned).  routes must hold 3 entries.  A
+ * diagnostic, no counterpart in the reference. */
 int dr_csr_routes(dr_csr* m, int64_t* routes);
 int dr_csr_free(dr_csr* m);
 
