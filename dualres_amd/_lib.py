@@ -108,6 +108,7 @@ SIGNATURES = {
     "dr_profile_kernels": [_P, _D, C.c_int, C.POINTER(C.c_int), _I64],
     "dr_kriging_build": [_D, C.POINTER(C.c_int), _F, _D, C.POINTER(C.c_int), _F, _D, C.c_double, C.c_int,
                          C.POINTER(_P)],
+    "dr_kriging_build_bytes": [_F, C.c_double, C.c_int64, C.c_int64, _I64, _I64],
     "dr_csr_info": [_P, _I64, _I64, _I64, _I64],
     "dr_csr_solver_counts": [_P, _I64, _I64],
     "dr_csr_routes": [_P, _I64],

@@ -1176,31 +1176,44 @@ __global__ void k_compact_rows(int n_rows, const long* __restrict__ rp, const lo
   }
 }
 
+// device bytes that this thread's build holds, and the most so far
+struct Held { long now = 0, peak = 0; };
+thread_local Held held;
+
 template <typename T>
 struct DBuf {
   T* p = nullptr;
+  size_t bytes = 0;
   DBuf() = default;
   explicit DBuf(size_t n) { alloc(n); }
   DBuf(const DBuf&) = delete;
   DBuf& operator=(const DBuf&) = delete;
-  DBuf(DBuf&& o) noexcept : p(o.p) { o.p = nullptr; }
+  DBuf(DBuf&& o) noexcept : p(o.p), bytes(o.bytes) { o.p = nullptr; }
   DBuf& operator=(DBuf&& o) noexcept {
     if (this != &o) {
-      if (p) (void)hipFree(p);
+      release();
       p = o.p;
+      bytes = o.bytes;
       o.p = nullptr;
     }
     return *this;
   }
-  ~DBuf() { if (p) (void)hipFree(p); }
-  void alloc(size_t n) {
-    if (p) (void)hipFree(p);
+  ~DBuf() { release(); }
+  void release() {
+    if (!p) return;
+    (void)hipFree(p);
     p = nullptr;
-    if (n == 0) n = 1;
-    if (hipMalloc((void**)&p, n * sizeof(T)) != hipSuccess) {
+    held.now -= (long)bytes;
+  }
+  void alloc(size_t n) {
+    release();
+    bytes = std::max<size_t>(n, 1) * sizeof(T);
+    if (hipMalloc((void**)&p, bytes) != hipSuccess) {
       p = nullptr;
       throw Error(DR_ENOMEM, "hipMalloc failed in kriging build");
     }
+    held.now += (long)bytes;
+    held.peak = std::max(held.peak, held.now);
   }
   void up(const T* h, size_t n, hipStream_t s) { DR_HIP(hipMemcpyAsync(p, h, n * sizeof(T), hipMemcpyHostToDevice, s)); }
   void down(T* h, size_t n, hipStream_t s) { DR_HIP(hipMemcpyAsync(h, p, n * sizeof(T), hipMemcpyDeviceToHost, s)); }
@@ -1216,6 +1229,7 @@ struct KrigingCSR {
   long n_batches = 0;  // batches of systems factorised directly, Cholesky and LU
   bool inverse_built = false;  // K^-1 was computed
   long n_inverse = 0;          // unique systems solved through it
+  long peak = 0;               // device bytes held at most
   std::vector<int64_t> rp;
   DBuf<int32_t> cols;
   DBuf<double> vals;
@@ -1230,25 +1244,26 @@ static float norm3f(const float* v) {
   return sqrt_rn(s);
 }
 
-KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], const double* st, const int sdims[3],
-                         const float qs[16], const double theta[3], double radius, int device) {
-  DR_REQUIRE(hr && st && hd && sdims && qh && qs && theta, DR_ELOGIC, "kriging_build: null argument");
-  DR_REQUIRE(radius >= 0, DR_EDOMAIN, "neighborhood_perturbation: radius cannot be negative");
-  DR_HIP(hipSetDevice(device));
-  const int nx = hd[0], ny = hd[1], nz = hd[2];
-  const long nvox = (long)nx * ny * nz;
-  // neighbourhood offsets (kriging_matrix.h:63-106)
-  float vd[3];
+constexpr int kMaxOffsets = 5000;
+// device bytes of a batch's or slab's factors, of each of a slab's four arrays
+// of rows, and systems of a batch
+constexpr double kFactorBytes = 6.0e9, kRowBytes = 1.5e9;
+constexpr long kBatchMax = 16384;
+
+// voxel steps along the axes that the neighbourhood reaches
+static void reach(const float qh[16], double radius, double r[3]) {
   for (int c = 0; c < 3; ++c) {
     float s = 0.0f;
-    for (int r = 0; r < 4; ++r) s += qh[4 * r + c] * qh[4 * r + c];
-    vd[c] = sqrt_rn(s);
+    for (int i = 0; i < 4; ++i) s += qh[4 * i + c] * qh[4 * i + c];
+    r[c] = (double)((float)radius / sqrt_rn(s));
   }
+}
+// neighbourhood offsets P and their displacements X (kriging_matrix.h:63-106)
+static void neighbourhood(const float qh[16], double radius, std::vector<int>& P, std::vector<float>& X) {
+  double r[3];
+  reach(qh, radius, r);
   const float rad = (float)radius;
-  int rng[3];
-  for (int c = 0; c < 3; ++c) rng[c] = (int)(rad / vd[c]);
-  std::vector<int> P;
-  std::vector<float> X;
+  const int rng[3] = {(int)r[0], (int)r[1], (int)r[2]};
   for (int z = -rng[2]; z <= rng[2]; ++z)
     for (int y = -rng[1]; y <= rng[1]; ++y)
       for (int x = -rng[0]; x <= rng[0]; ++x) {
@@ -1260,9 +1275,46 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
           X.insert(X.end(), {xx[0], xx[1], xx[2]});
         }
       }
+}
+
+// Offsets of the neighbourhood (more than kMaxOffsets: no build) and device
+// bytes that a build of at most n_rows rows on nvox fine voxels holds at its
+// peak, whichever way its systems go.
+static void build_bytes(const float qh[16], double radius, double n_rows, double nvox, int64_t* n_offsets,
+                        int64_t* bytes) {
+  double r[3], box = 1.0;
+  reach(qh, radius, r);
+  for (int c = 0; c < 3; ++c) box *= 2.0 * std::floor(r[c]) + 1.0;
+  std::vector<int> P;
+  std::vector<float> X;
+  if (box <= 1e6) neighbourhood(qh, radius, P, X);  // a larger box has too many offsets
+  else P.resize(3 * ((size_t)kMaxOffsets + 1));
+  const double nP = (double)P.size() / 3, ld = std::ceil(nP / NB) * NB, nnz = n_rows * nP;
+  const double image = 5.0 * nvox + 80.0 * n_rows + 1e6;   // presence, index; per row; small tables
+  const double entries = 20.0 * nnz;                       // column, offset, k', solution
+  const double matrices = 4.0 * nP * nP + 16.0 * ld * ld;  // K (float32, float64), K^-1
+  const double inverse = 16.0 * ld * ld;                   // its factor, the factor's inverse
+  const double factors = std::min(kFactorBytes, 8.0 * n_rows * ld * ld);  // of a slab or of a direct batch
+  const double slab = 2.0 * nnz + 4.0 * std::min(kRowBytes, 8.0 * (n_rows + NB) * ld);  // absent offsets, rows
+  const double direct = 8.0 * std::min<double>(n_rows, kBatchMax) * ld + 20.0 * nnz;  // right-hand sides; W, W compacted
+  *n_offsets = (int64_t)nP;
+  *bytes = (int64_t)(image + entries + matrices + std::max(inverse, factors + std::max(slab, direct)));
+}
+
+KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], const double* st, const int sdims[3],
+                         const float qs[16], const double theta[3], double radius, int device) {
+  DR_REQUIRE(hr && st && hd && sdims && qh && qs && theta, DR_ELOGIC, "kriging_build: null argument");
+  DR_REQUIRE(radius >= 0, DR_EDOMAIN, "neighborhood_perturbation: radius cannot be negative");
+  DR_HIP(hipSetDevice(device));
+  held = Held{};
+  const int nx = hd[0], ny = hd[1], nz = hd[2];
+  const long nvox = (long)nx * ny * nz;
+  std::vector<int> P;
+  std::vector<float> X;
+  neighbourhood(qh, radius, P, X);
   const int nP = (int)(P.size() / 3);
   DR_REQUIRE(nP > 0, DR_ELOGIC, "neighborhood_perturbation: no perturbations within radius");
-  DR_REQUIRE(nP <= 5000, DR_ELOGIC, "get_sparse_kriging_array_data: neighborhood >5e3 voxels");
+  DR_REQUIRE(nP <= kMaxOffsets, DR_ELOGIC, "get_sparse_kriging_array_data: neighborhood >5e3 voxels");
   Geo g{};
   g.tau2 = (double)(float)theta[0];
   g.psi = (double)(float)theta[1];
@@ -1498,7 +1550,6 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
   // 305 20.2 / 19.3 / 18.8 / 17.7 / 19.1; by Cholesky 638 of 1,357 52 / 37 / 24 /
   // 25 / 25, 1,728 63 / 62 / 53 / 47 / 51.
   constexpr int kBatchMin = 512;
-  const double budget = 6.0e9;  // bytes of factor scratch per batch
   DBuf<double> d_A, d_b;
   DBuf<SysDesc> d_sd;
   size_t capA = 0, capB = 0, capS = 0;
@@ -1511,7 +1562,7 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
     while (pos < uids.size()) {
       const int np = cdiv(cnt[urow[uids[pos]]], NB) * NB;
       const long per = (long)np * np * 8;
-      const int bmax = (int)std::max<long>(1, std::min<long>(16384, (long)(budget / per)));
+      const int bmax = (int)std::max<long>(1, std::min<long>(kBatchMax, (long)(kFactorBytes / per)));
       std::vector<SysDesc> sd;
       const size_t first = pos;
       while (pos < uids.size() && (int)sd.size() < bmax &&
@@ -1579,7 +1630,7 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
     size_t e1 = e0;
     for (; e1 < order.size(); ++e1) {
       const int u = order[e1], n = cnt[urow[u]], m = msize(u), np = cdiv(m, NB) * NB;
-      if (e1 > e0 && ((double)(fac + (long)np * np) * 8 > budget || (double)(ed.size() + NB) * ld * 8 > 1.5e9)) break;
+      if (e1 > e0 && ((double)(fac + (long)np * np) * 8 > kFactorBytes || (double)(ed.size() + NB) * ld * 8 > kRowBytes)) break;
       const bool dir = n < nP - n;
       if (m > 0) {
         fd.push_back(FacDesc{m, dir ? -1 : (int)ed.size(), dir ? rp[urow[u]] : dl, fac, usol[u]});
@@ -1703,6 +1754,7 @@ KrigingCSR kriging_build(const double* hr, const int hd[3], const float qh[16], 
     DR_HIP(hipStreamSynchronize(s));
   }
   (void)oobv;
+  out.peak = held.peak;
   return out;
 }
 
@@ -1721,6 +1773,15 @@ int dr_kriging_build(const double* hr, const int hr_dims[3], const float q_hr[16
     DR_REQUIRE(out, DR_ELOGIC, "dr_kriging_build: null output");
     auto* c = new dr_csr{drh::kriging_build(hr, hr_dims, q_hr, std_img, std_dims, q_std, theta, radius, device)};
     *out = c;
+  });
+}
+
+int dr_kriging_build_bytes(const float q_hr[16], double radius, int64_t n_rows, int64_t n_voxels, int64_t* n_offsets,
+                           int64_t* bytes) {
+  return drh::guarded([&] {
+    DR_REQUIRE(q_hr && n_offsets && bytes, DR_ELOGIC, "dr_kriging_build_bytes: null argument");
+    DR_REQUIRE(!(radius < 0), DR_EDOMAIN, "neighborhood_perturbation: radius cannot be negative");
+    drh::build_bytes(q_hr, radius, (double)n_rows, (double)n_voxels, n_offsets, bytes);
   });
 }
 
@@ -1748,6 +1809,7 @@ int dr_csr_routes(dr_csr* m, int64_t* routes) {
     routes[0] = m->m.n_batches;
     routes[1] = m->m.inverse_built ? 1 : 0;
     routes[2] = m->m.n_inverse;
+    routes[3] = m->m.peak;
   });
 }
 

@@ -99,21 +99,15 @@ int64_t estimate_request_bytes(const ServeRequest& r) {
   std::vector<int32_t> flat;
   flat.reserve(3 * ijk.size());
   for (const auto& v : ijk) flat.insert(flat.end(), {v[0], v[1], v[2]});
-  int64_t n_s = 0, P = 0;
+  int64_t n_s = 0, P = 0, build = 0;
   if (r.n_datasets == 2) {
     for (double v : r.sr) n_s += present(v) ? 1 : 0;
-    const auto vd = voxel_dimensions(r.qh);
-    const double rad = default_neighborhood(r);
-    P = 1;
-    for (int a = 0; a < 3; ++a) P *= 2 * (int64_t)std::floor(rad / std::max(1e-6f, vd[a])) + 1;
+    check(dr_kriging_build_bytes(r.qh.data(), default_neighborhood(r), n_s, (int64_t)r.hr.size(), &P, &build));
   }
   const dr_config cfg = make_config(r, 0);
   int64_t b = 0;
   check(dr_estimate_bytes(&cfg, flat.data(), (int64_t)ijk.size(), n_s, n_s * P, &b));
-  if (r.n_datasets == 2) {  // kriging build: patterns, systems (batched to <= 6e9 bytes), CSR
-    const double sys = std::min(6.5e9, 1.1 * (double)n_s * (double)P * (double)P * 8.0);
-    b += (int64_t)sys + n_s * P * 24;
-  }
+  b += build;
   return b;
 }
 

@@ -34,12 +34,22 @@ def kriging_build(hr, q_hr, std, q_std, theta, radius, device=0, return_info=Fal
         L.check(lib.dr_csr_copy(h, L.iptr64(rp), L.iptr32(cols), L.dptr(vals)))
         nch, nlu = C.c_int64(), C.c_int64()
         L.check(lib.dr_csr_solver_counts(h, C.byref(nch), C.byref(nlu)))
-        routes = np.zeros(3, dtype=np.int64)
+        routes = np.zeros(4, dtype=np.int64)
         L.check(lib.dr_csr_routes(h, L.iptr64(routes)))
     finally:
         lib.dr_csr_free(h)
     W = sp.csr_matrix((vals, cols, rp), shape=(nrow.value, ncol.value))
     if return_info:
         return W, {"n_unique_solves": nu.value, "nnz": nnz.value, "n_cholesky": nch.value, "n_lu": nlu.value,
-                   "n_batches": int(routes[0]), "inverse_built": bool(routes[1]), "n_inverse": int(routes[2])}
+                   "n_batches": int(routes[0]), "inverse_built": bool(routes[1]), "n_inverse": int(routes[2]),
+                   "peak_bytes": int(routes[3])}
     return W
+
+
+def kriging_build_bytes(q_hr, radius, n_rows, n_voxels):
+    """(offsets of the neighbourhood, bound of the device bytes a build holds at its peak)."""
+    n, b = C.c_int64(), C.c_int64()
+    q = np.ascontiguousarray(q_hr, dtype=np.float32).reshape(16)
+    L.check(L.load().dr_kriging_build_bytes(L.fptr(q), float(radius), int(n_rows), int(n_voxels), C.byref(n),
+                                            C.byref(b)))
+    return n.value, b.value

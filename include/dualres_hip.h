@@ -263,6 +263,12 @@ typedef struct dr_csr dr_csr;
 int dr_kriging_build(const double* hr, const int hr_dims[3], const float q_hr[16],
                      const double* std_img, const int std_dims[3], const float q_std[16],
                      const double theta[3], double radius, int device, dr_csr** out);
+/* Offsets of the neighbourhood that a build with this fine qform and radius
+ * takes (more than 5,000: it is refused), and an upper bound of the device bytes it
+ * holds at its peak with n_rows coarse rows on n_voxels fine voxels.  Needs no
+ * device. */
+int dr_kriging_build_bytes(const float q_hr[16], double radius, int64_t n_rows, int64_t n_voxels, int64_t* n_offsets,
+                           int64_t* bytes);
 int dr_csr_info(dr_csr* m, int64_t* nrow, int64_t* ncol, int64_t* nnz, int64_t* n_unique_solves);
 int dr_csr_copy(dr_csr* m, int64_t* rowptr, int32_t* cols, double* vals);
 /* Unique systems solved by Cholesky and by the pivoted LU that takes the
@@ -273,8 +279,9 @@ int dr_csr_solver_counts(dr_csr* m, int64_t* n_cholesky, int64_t* n_lu);
 /* How the systems were worked on: routes[0] = batches factorised directly, by
  * Cholesky and by LU; [1] whether the inverse of the whole neighbourhood's kernel
  * matrix was computed; [2] the unique systems solved through it (0 although it
- * was computed: it was too ill conditioned).  routes must hold 3 entries.  A
- * diagnostic, no counterpart in the reference. */
+ * was computed: it was too ill conditioned); [3] the device bytes that the build
+ * held at its peak.  routes must hold 4 entries.  A diagnostic, no counterpart in
+ * the reference. */
 int dr_csr_routes(dr_csr* m, int64_t* routes);
 int dr_csr_free(dr_csr* m);
 
