@@ -74,6 +74,7 @@ SIGNATURES = {
     "dr_add_data_to_mu": [_P],
     "dr_w_layout": [_P, C.c_int],
     "dr_w_stats": [_P, _I64],
+    "dr_routes": [_P, _I64],
     "dr_set_output_indices": [_P, _I32, C.c_int64],
     "dr_get_mu_output": [_P, _D, C.c_int64],
     "dr_estimate_bytes": [C.POINTER(dr_config), _I32, C.c_int64, C.c_int64, C.c_int64, _I64],

@@ -151,6 +151,8 @@ struct ChainBase {
   bool use_cls = false;    // class-stencil W kernels active
   bool force_csr = false;  // keep the plain CSR kernels (tests)
   int64_t wstats[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  int64_t wlines[4] = {0, 0, 0, 0};  // dr_routes [0] to [3]
+  int lik_route = -1;                // kernels of the last likelihood: 0 separate passes, 1 by rows, 2 by planes
   // cached energies of the current state A
   bool stats_valid = false;
   double prior_sum = 0.0, sse_h = 0.0, sse_s = 0.0;
@@ -1494,6 +1496,10 @@ struct Chain : public ChainBase {
     wstats[7] = LT[0] * LT[1] * LT[2];
     wstats[8] = Tt[0] * Tt[1] * Tt[2];
     wstats[9] = (int64_t)frow.size();
+    wlines[0] = ws.sxm;
+    wlines[1] = ws.sxm ? ws.nc : 0;
+    wlines[2] = ws.sx;
+    wlines[3] = ws.sx ? ws.mc : 0;
     return true;
   }
 
@@ -1537,6 +1543,7 @@ struct Chain : public ChainBase {
       std::vector<T> ys(n_s);
       for (long i = 0; i < n_s; ++i) ys[i] = (T)Ys[i];
       DR_HIP(hipMemcpyAsync(Ysd.p, ys.data(), n_s * sizeof(T), hipMemcpyHostToDevice, stream));
+      std::fill(wlines, wlines + 4, 0);
       use_cls = !force_csr && build_stencil(rp, cols, vals);
       if (!use_cls) {
         // transposed CSR for W^T v, rows ascending within each column
@@ -1720,7 +1727,9 @@ struct Chain : public ChainBase {
   // transformed back into T1.  A single-resolution residual is local to a row
   // and takes one kernel on T2 in place, which writes mu to R only if keep.
   void likelihood(T* R, int slot_h, int slot_s, bool keep) {
+    lik_route = 2;
     if (cfg.n_datasets == 1 && planes(row_args(keep ? R : nullptr), residual(R, slot_h), slot_h)) return;
+    lik_route = 1;
     if (cfg.n_datasets == 1 && lines_ok(0, P_XI) && lines_ok(0, P_XF)) {
       y_inverse();
       if (const int g = rows_residual(M[0] / 2, row_args(keep ? R : nullptr), residual(R, slot_h), stream)) {
@@ -1735,6 +1744,7 @@ struct Chain : public ChainBase {
     } else {
       c2r_yx(R);
     }
+    lik_route = 0;
     w_products(R, slot_s);
     r2c_xy(residual(R, slot_h), slot_h);
   }
@@ -2470,6 +2480,13 @@ int dr_w_layout(dr_chain* c, int force_csr) {
   return guarded([&] { c->impl->force_csr = force_csr != 0; });
 }
 
+int dr_routes(dr_chain* c, int64_t* routes) {
+  return guarded([&] {
+    DR_REQUIRE(c && routes, DR_ELOGIC, "dr_routes: null argument");
+    for (int i = 0; i < 4; ++i) routes[i] = c->impl->wlines[i];
+    routes[4] = c->impl->lik_route;
+  });
+}
 int dr_w_stats(dr_chain* c, int64_t* stats) {
   return guarded([&] {
     auto& k = *c->impl;

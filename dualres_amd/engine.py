@@ -107,6 +107,13 @@ class Chain:
                 "touched_voxels": int(st[6]), "interior_tiles": int(st[7]), "tile_cells": int(st[8]),
                 "tile_voxels": int(st[9]), "far_rows": int(st[10])}
 
+    def routes(self):
+        """Which kernels the W products and the last likelihood take (dr_routes)."""
+        r = np.zeros(5, dtype=np.int64)
+        L.check(self._lib.dr_routes(self._h, L.iptr64(r)))
+        return {"w_mu_step": int(r[0]), "w_mu_chunks": int(r[1]), "wt_v_step": int(r[2]), "wt_v_chunks": int(r[3]),
+                "likelihood": {2: "planes", 1: "rows", 0: "passes", -1: None}[int(r[4])]}
+
     def add_data_to_mu(self):
         L.check(self._lib.dr_add_data_to_mu(self._h))
 

@@ -123,6 +123,12 @@ int dr_w_layout(dr_chain* c, int force_csr);
  * per tile; [10] far rows (boundary rows too wide to pack, counted in [3]).
  * stats must hold 11 entries. */
 int dr_w_stats(dr_chain* c, int64_t* stats);
+/* Which kernels run, a diagnostic: [0] lattice step by which W mu of the stencil
+ * rows goes by stencil lines (0: by another kernel) and [1] the chunks of 4 taps
+ * of its longest line; [2], [3] the same of W^T v; [4] the last update's
+ * likelihood: 2 by whole planes, 1 in one kernel of rows, 0 by separate passes,
+ * -1 none yet.  routes must hold 5 entries. */
+int dr_routes(dr_chain* c, int64_t* routes);
 
 /* mcmc_summary<T> (gaussian_process_model.h:191-224) kept on the device:
  * dr_summary_update adds mu, mu^2 and |mu| / max(max|mu|, 1e-6) of the
