@@ -403,6 +403,17 @@ struct Chain : public ChainBase {
   }
   double* pslot(int s) { return part.p + (long)s * pstride; }
 
+  // the columns that pad the last block of a spectral array, which nothing
+  // writes afterwards (the whole block: its columns are written before they are
+  // read).  Whole arrays instead took 0.35 ms of 6.8 to create a 256x512x256
+  // chain in float64.
+  template <typename V>
+  void zero_padding(DevBuf<V>& b) {
+    const Spec<T> sp = spec();
+    const long block = (long)Spec<T>::C * sp.M2;
+    if (sp.NB % Spec<T>::C) DR_HIP(hipMemsetAsync(b.p + (Ns - block), 0, block * sizeof(V), stream));
+  }
+
   // ------------------------------------------------------------ build
   void build() override {
     DR_HIP(hipSetDevice(cfg.device));
@@ -442,10 +453,10 @@ struct Chain : public ChainBase {
     muA.alloc(Ns);
     muB.alloc(Ns);
     p.alloc(Ns);
-    invlam.zero(stream);  // the padding stays 0
-    lam.zero(stream);
-    muA.zero(stream);
-    muB.zero(stream);
+    zero_padding(invlam);
+    zero_padding(lam);
+    zero_padding(muA);
+    zero_padding(muB);
     p.zero(stream);
     T1.alloc(Nh);
     T2.alloc(Nh);
@@ -453,8 +464,8 @@ struct Chain : public ChainBase {
       miA.alloc(Ns);
       miB.alloc(Ns);
       pim.alloc(Ns);
-      miA.zero(stream);
-      miB.zero(stream);
+      zero_padding(miA);
+      zero_padding(miB);
       pim.zero(stream);
     }
     int r[3];
