@@ -196,7 +196,7 @@ template <typename T> constexpr int line_cap() { return sizeof(T) == 4 ? 20 : 10
 template <typename T> constexpr int line_cols(int nj) { return nj < 16 || (sizeof(T) == 4 && nj <= 64) ? 16 : 8; }
 template <typename T, int M, int CAP> struct LineShape {
   using Plan = LinePlan<M, CAP>;
-  static constexpr int TB = line_cols<T>(Plan::nj), NT = Plan::nj * TB;
+  static constexpr int TB = line_cols<T>(Plan::nj), NT = Plan::nj * TB, COLS = TB;
   static_assert(NT <= 1024, "workgroup");
 };
 template <typename T, int M> using StridedShape = LineShape<T, M, kCapStrided>;
@@ -387,7 +387,7 @@ k_zkick(const cx<T>* tw, int nb, int n_in, const cx<T>* T1, EpiMomentum<T> em) {
 // from the cache, in place of an exchange.
 template <typename T, int Mh> struct RowShape {
   using Plan = LinePlan<Mh, line_cap<T>()>;
-  static constexpr int RW = Plan::nj >= 64 ? 1 : 64 / Plan::nj, NT = RW * Plan::nj;
+  static constexpr int RW = Plan::nj >= 64 ? 1 : 64 / Plan::nj, NT = RW * Plan::nj, COLS = RW;
   static constexpr int R1 = Plan::P.r[0];
   // a pad slot after every R1 elements where R1 is even: the first stage
   // writes at stride R1, which then hits every bank
@@ -827,30 +827,72 @@ __global__ void __launch_bounds__((StridedShape<double, M>::NT)) k_corr_z(CorrZ 
 }
 
 // ---------------------------------------------------------------- host side
-// Each returns the number of workgroups launched, 0 when no kernel was built
-// for the length (the caller then takes the kernels of dr_fft.hpp).
-#define DR_LINE_API(T)                                                                                             \
-  int lines_inverse(int M, const LineArgs<T>& a, hipStream_t s);                                                   \
-  int lines_forward(int M, const LineArgs<T>& a, hipStream_t s);                                                   \
-  int lines_z(int M, const cx<T>* tw, int nb, int n_in, int n_out, cx<T>* T1, const MidLeapfrog<T>& mid,           \
-              hipStream_t s);                                                                                      \
-  int lines_z_kick(int M, const cx<T>* tw, int nb, int n_in, const cx<T>* T1, const EpiMomentum<T>& em,            \
-                   hipStream_t s);                                                                                 \
-  int rows_c2r(int Mh, const RowArgs<T>& a, hipStream_t s);                                                        \
-  int rows_r2c(int Mh, const RowArgs<T>& a, const LoadResidual<T>& res, hipStream_t s);                            \
-  int rows_residual(int Mh, const RowArgs<T>& a, const LoadResidual<T>& res, hipStream_t s);                        \
-  int plane_residual(int Mh, int MY, int nz, const PlaneArgs<T>& a, const LoadResidual<T>& res, hipStream_t s);
-DR_LINE_API(float)
-DR_LINE_API(double)
-#undef DR_LINE_API
-int rows_mask(int Mh, const MaskRows& a, hipStream_t s);
-int lines_corr(int M, const CorrZ& a, hipStream_t s);
-
+// The lengths with kernels and the part of them an object of dr_lines.hip holds.
 #define DR_LINE_LENGTHS(X)                                                                                           \
   X(8) X(10) X(12) X(14) X(16) X(18) X(20) X(24) X(28) X(30) X(32) X(36) X(40) X(42) X(48) X(50) X(54) X(56) X(60)    \
   X(64) X(70) X(72) X(80) X(84) X(90) X(96) X(98) X(100) X(108) X(112) X(120) X(126) X(128) X(140) X(144) X(150)      \
   X(160) X(162) X(168) X(180) X(192) X(196) X(200) X(210) X(216) X(224) X(240) X(250) X(252) X(256) X(270) X(280)     \
   X(288) X(294) X(300) X(320) X(324) X(336) X(350) X(360) X(378) X(384) X(392) X(400) X(420) X(432) X(448) X(450)     \
   X(480) X(486) X(490) X(500) X(504) X(512)
+constexpr int kLineParts = 6;
+constexpr int line_part(int M) { return M <= 48 ? 0 : M <= 96 ? 1 : M <= 150 ? 2 : M <= 240 ? 3 : M <= 336 ? 4 : 5; }
+template <class F>
+inline int with_line_part(int M, F&& f) {
+  switch (line_part(M)) {
+    case 0: return f(std::integral_constant<int, 0>{});
+    case 1: return f(std::integral_constant<int, 1>{});
+    case 2: return f(std::integral_constant<int, 2>{});
+    case 3: return f(std::integral_constant<int, 3>{});
+    case 4: return f(std::integral_constant<int, 4>{});
+    default: return f(std::integral_constant<int, 5>{});
+  }
+}
+#define DR_PART(M, call) with_line_part(M, [&](auto p) { constexpr int P = decltype(p)::value; return call; })
+
+// Each returns the number of workgroups launched, 0 when no kernel was built
+// for the length (the caller then takes the kernels of dr_fft.hpp).
+#define DR_LINE_API(T)                                                                                               \
+  template <int P, bool INV> int lines_strided_part(int M, const LineArgs<T>& a, hipStream_t s);                     \
+  template <int P> int lines_z_part(int M, const cx<T>* tw, int nb, int n_in, int n_out, cx<T>* T1,                  \
+                                    const MidLeapfrog<T>& mid, hipStream_t s);                                       \
+  template <int P> int lines_z_kick_part(int M, const cx<T>* tw, int nb, int n_in, const cx<T>* T1,                  \
+                                         const EpiMomentum<T>& em, hipStream_t s);                                   \
+  template <int P> int rows_c2r_part(int Mh, const RowArgs<T>& a, hipStream_t s);                                    \
+  template <int P> int rows_r2c_part(int Mh, const RowArgs<T>& a, const LoadResidual<T>& res, hipStream_t s);        \
+  template <int P> int rows_residual_part(int Mh, const RowArgs<T>& a, const LoadResidual<T>& res, hipStream_t s);   \
+  inline int lines_inverse(int M, const LineArgs<T>& a, hipStream_t s) {                                             \
+    return DR_PART(M, (lines_strided_part<P, true>(M, a, s)));                                                       \
+  }                                                                                                                  \
+  inline int lines_forward(int M, const LineArgs<T>& a, hipStream_t s) {                                             \
+    return DR_PART(M, (lines_strided_part<P, false>(M, a, s)));                                                      \
+  }                                                                                                                  \
+  inline int lines_z(int M, const cx<T>* tw, int nb, int n_in, int n_out, cx<T>* T1, const MidLeapfrog<T>& mid,      \
+                     hipStream_t s) {                                                                                \
+    return DR_PART(M, lines_z_part<P>(M, tw, nb, n_in, n_out, T1, mid, s));                                          \
+  }                                                                                                                  \
+  inline int lines_z_kick(int M, const cx<T>* tw, int nb, int n_in, const cx<T>* T1, const EpiMomentum<T>& em,       \
+                          hipStream_t s) {                                                                           \
+    return DR_PART(M, lines_z_kick_part<P>(M, tw, nb, n_in, T1, em, s));                                             \
+  }                                                                                                                  \
+  inline int rows_c2r(int Mh, const RowArgs<T>& a, hipStream_t s) {                                                  \
+    return DR_PART(2 * Mh, rows_c2r_part<P>(Mh, a, s));                                                              \
+  }                                                                                                                  \
+  inline int rows_r2c(int Mh, const RowArgs<T>& a, const LoadResidual<T>& res, hipStream_t s) {                      \
+    return DR_PART(2 * Mh, rows_r2c_part<P>(Mh, a, res, s));                                                         \
+  }                                                                                                                  \
+  inline int rows_residual(int Mh, const RowArgs<T>& a, const LoadResidual<T>& res, hipStream_t s) {                 \
+    return DR_PART(2 * Mh, rows_residual_part<P>(Mh, a, res, s));                                                    \
+  }                                                                                                                  \
+  int plane_residual(int Mh, int MY, int nz, const PlaneArgs<T>& a, const LoadResidual<T>& res, hipStream_t s);
+DR_LINE_API(float)
+DR_LINE_API(double)
+#undef DR_LINE_API
+template <int P> int rows_mask_part(int Mh, const MaskRows& a, hipStream_t s);
+template <int P> int lines_corr_part(int M, const CorrZ& a, hipStream_t s);
+inline int rows_mask(int Mh, const MaskRows& a, hipStream_t s) {
+  return DR_PART(2 * Mh, rows_mask_part<P>(Mh, a, s));
+}
+inline int lines_corr(int M, const CorrZ& a, hipStream_t s) { return DR_PART(M, lines_corr_part<P>(M, a, s)); }
+#undef DR_PART
 
 }  // namespace drh
