@@ -111,8 +111,8 @@ template <typename T> struct MidLeapfrog {
   // thread only, so a thread may fetch its modes' state early
   struct State { cx<T> x, p; T il; };
   template <class I> __device__ __forceinline__ State fetch_at(I i) const {
-    // 1/lambda keeps cached loads: a 16-column tile reads half of each of its
-    // 128-byte lines, and the neighbouring tile the other half
+    // 1/lambda keeps cached loads: two neighbouring kz of a column block share
+    // a 128-byte line, and other lanes of the workgroup read the other half
     return State{nt_ld(X + i), nt_ld(p + i), invlam[i]};
   }
   // mode i of column b; write = false leaves memory and the sum alone

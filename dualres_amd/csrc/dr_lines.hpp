@@ -649,6 +649,7 @@ template <typename T, int Mh, int MY> struct PlaneShape {
   using Plan = LinePlan<MY, 16>;
   using Row = RowShape<T, Mh>;
   static constexpr int LY = kPlaneNT / Plan::nj, LX = kPlaneNT / Row::Plan::nj;
+  static_assert(kPlaneNT % Plan::nj == 0 && kPlaneNT % Row::Plan::nj == 0, "whole lines");
   static constexpr int EY = MY * LY, EX = LX * Row::P;
   static constexpr int E = EY > EX ? EY : EX;    // exchange buffer
   static constexpr int rows = MY / 2 + 1;        // region rows a torus of twice the data holds
